@@ -701,9 +701,9 @@ __global__ __launch_bounds__(NT) void k_attention_gqa(const int64_t* __restrict_
     }
   }
   __syncthreads();
-  if (wave <= HB) {   // waves 0 .. HB - 1: RoPE + qrow of the query heads, wave HB: of the new key
+  for (int hw = wave; hw <= HB; hw += NW) {   // heads 0 .. HB - 1: RoPE + qrow of the query heads, HB: of the new key
     const int half = hd >> 1;
-    const int64_t* yy = y[wave];
+    const int64_t* yy = y[hw];
     int64_t z[2];
     int64_t m = 0;
 #pragma unroll
@@ -726,11 +726,11 @@ __global__ __launch_bounds__(NT) void k_attention_gqa(const int64_t* __restrict_
       if (j < hd) {
         const int64_t w = shr64(z[i], q);
         const int32_t wc = (int32_t)(w > 32767 ? 32767 : (w < -32767 ? -32767 : w));
-        if (wave < HB) qs16[wave][j] = (int16_t)wc;
+        if (hw < HB) qs16[hw][j] = (int16_t)wc;
         else kn[j] = wc;
       }
     }
-    if (lane == 0) shq[wave] = q;
+    if (lane == 0) shq[hw] = q;
   }
   __syncthreads();
   const int skn = shq[HB];
