@@ -47,6 +47,7 @@ SIGNATURES = {
     "exact_attention": [P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, I32, I32, P],
     "exact_attention_qkv": [P, P, P, P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, I32, I32, P],
     "exact_attention_qkv_split": [P, P, P, P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, I32, I32, I32, P],
+    "exact_attention_decode": [P, P, P, P, P, P, P, P, P, P, P, P, P, I32, P, I64, I32, I32, I32, I32, I32, I32, P],
     "exact_attention_prefill": [P, P, P, P, P, I32, P, P, P, P, P, I64, I32, I32, I32, I32, I32, I32, I32, P],
     "exact_embed": [P, P, P, I32, I32, I32, P],
     "exact_embed_table": [P, P, P, I32, I32, P],
@@ -68,6 +69,7 @@ SIGNATURES = {
     "exact_moe_combine": [P, P, P, P, P, P, P, P, I32, I32, I32, I32, P],
 }
 OTHER = {"exact_version": ([], ctypes.c_int), "exact_last_error": ([], ctypes.c_char_p),
+         "exact_attention_decode_workspace": ([I32, I32, I32, I32, I32], ctypes.c_int64),
          "exact_attention_prefill_workspace": ([I32, I32, I32, I32, I32], ctypes.c_int64)}
 ERRORS = {1: "bad argument", 2: "unsupported size", 3: "HIP launch error"}
 

@@ -225,6 +225,7 @@ class Workspace:
         self.seq = None   # (slot, keys) when the rows are one sequence's consecutive positions (prefill)
         self.h = None     # (R, I) SwiGLU values when the gate|up totals must stay intact (trace capture)
         self.hsh = None   # (R, SI) SwiGLU values of the MoE shared expert (decode rows)
+        self.att_work = None   # of decode attention split over the keys
         self.eh = self.part_eh = None   # the routed experts' SwiGLU values per pair and their slice bit lengths
         self.I = I
         # int16 GEMM rows (prefill above 16 rows): the producers also write their rows' int8 digit rows, which the
@@ -296,6 +297,12 @@ class TModel:
             self._pws = (R, ops.prefill_workspace(R, self.cfg.H, self.cfg.KV, self.cfg.hd, self.Smax, self.dev))
         return self._pws[1]
 
+    def attention_work(self, ws):
+        if ws.att_work is None:
+            c = self.cfg
+            ws.att_work = ops.attention_work(ws.R, c.H, c.KV, c.hd, self.Smax, self.dev)
+        return ws.att_work
+
     def workspace(self, R):
         if R not in self._ws:
             self._ws[R] = Workspace(self.cfg, R, self.dev, self.nq, self.I, self.abits)
@@ -315,12 +322,14 @@ class TModel:
         return out
 
     # ---------------------------------------------------------------- one pass over R rows
-    def forward_rows(self, ws, want_logits=True, trace=None, independent=False, last_only=False):
+    def forward_rows(self, ws, want_logits=True, trace=None, independent=False, last_only=False, keys=None):
         """Runs the model on ws.ids with (slot, pos) per row; KV of each row is written into the cache
         at (slot, pos). Leaves logits in ws.logits and greedy ids in ws.next_ids (last_only: of the last row only, the
         others are left as they were; the final norm, the head and the argmax run on that row alone).
         independent: every row is a different sequence (decode), so no row attends to another row's new key and
         the q/k/v epilogue runs inside the attention launch.
+        keys: the positions the pass's longest row attends to, when the caller knows them (else the cache's): they decide
+        whether decode attention is split over the keys.
         trace: (TraceLayout, int64 device buffer): every linear's totals t are produced in the buffer's slots
         and left there (the buffer is zeroed first); the consumer kernels read them without clearing."""
         c, R, tab = self.cfg, ws.R, self.tab
@@ -341,10 +350,17 @@ class TModel:
         # launch at 8 rows
         xfuse = group and R <= self.QROW_FUSE_ROWS
         afuse = xfuse and ws.seq is None and (R == 1 or independent)
+        # decode attention over many positions: split over the keys, the q|k|v epilogue inside at any batch
+        keys = min(keys or self.Smax, self.Smax)
+        ksplit = (group and ws.seq is None and (R == 1 or independent)
+                  and keys >= ops.attention_keys_from(R, H, KV, hd, self.Smax))
+        if ksplit:
+            self.attention_work(ws)
         # batched decode rows (each its own sequence): the q|k|v epilogue inside the attention launch as well, whose
-        # totals the attention output's qrow launch then clears (caches of up to 256 positions: 8 threads per key)
+        # totals the attention output's qrow launch then clears (caches of up to 256 positions: 8 threads per key; longer
+        # ones while the (row, head) blocks fit one round: 8 rows of 28 heads at 301 positions 14.4 against 21.1 us)
         bfuse = (self.BATCH_ATTN and group and not xfuse and ws.seq is None and independent and hd % 64 == 0 and hd <= 128
-                 and self.Smax <= 256)
+                 and (self.Smax <= 256 or ksplit or R * H <= ops.ATT_ROUND_BLOCKS))
         # decode rows of dense int16 models: residual + RMSNorm + qrow run inside the GEMVs that consume them (q|k|v,
         # gate|up, head), which read one residual buffer and write the other
         nfuse = (afuse and self.abits == 15 and not c.moe and R <= ops.NORM_FUSE_ROWS and D <= self.NORM_FUSE_D
@@ -411,7 +427,7 @@ class TModel:
             nob = H   # bit lengths per row that attention leaves in ws.obits
             if afuse or bfuse:
                 ops.attention_qkv(t_qkv, s_qkv, b_qkv, tab.cos, tab.sin, ws.slot, ws.pos, cache, tab.exp, ws.att, H, KV, hd,
-                                  tab.inv, ws.obits, obn=self.ATT_SPLIT)
+                                  tab.inv, ws.obits, obn=self.ATT_SPLIT, keys=keys, work=ws.att_work)
                 nob = H * self.ATT_SPLIT
             else:
                 ops.qkv_rope_cache(t_qkv if group else ws.t_qkv, s_qkv, b_qkv, tab.cos, tab.sin, ws.slot, ws.pos, cache,
@@ -634,11 +650,11 @@ class TModel:
                 self._graphs.move_to_end(key)
                 g[0].replay()
             else:
-                self.forward_rows(ws, last_only=last_only)
+                self.forward_rows(ws, last_only=last_only, keys=p0 + T)
                 if graph:   # capture the same pass (capture records, it does not run the kernels again)
                     cg = torch.cuda.CUDAGraph()
                     with torch.cuda.graph(cg):
-                        self.forward_rows(ws, last_only=last_only)
+                        self.forward_rows(ws, last_only=last_only, keys=p0 + T)
                     self._graphs[key] = (cg, cache)   # the graph holds the cache's buffers
                     while len(self._graphs) > self.PREFILL_GRAPHS:
                         self._graphs.popitem(last=False)
@@ -667,7 +683,7 @@ class TModel:
         ws.pos.copy_(torch.arange(p0, p0 + T, dtype=I32))
         ws.seq = (slot, p0 + T) if T >= self.PREFILL_MIN_ROWS.get(self.cfg.hd, 1 << 30) else None
         try:
-            self.forward_rows(ws, trace=(layout, buf))
+            self.forward_rows(ws, trace=(layout, buf), keys=p0 + T)
         finally:
             ws.seq = None
         cache.n[slot] = p0 + T
@@ -683,7 +699,7 @@ class TModel:
         ws.pos.copy_(torch.tensor(cache.n[:B], dtype=I32))
         if max(cache.n[:B]) >= self.Smax:
             raise ExactError("cache full")
-        self.forward_rows(ws, independent=True)
+        self.forward_rows(ws, independent=True, keys=max(cache.n[:B]) + 1)
         for r in range(B):
             cache.n[r] += 1
         return ws.logits.clone(), ws.next_ids.clone()
@@ -810,14 +826,15 @@ class GraphDecoder:
         TraceRecorder with record() to copy and commit them."""
         self.tm, self.cache, self.B = tm, cache, B
         self.ws = tm.workspace(B)
-        self.graph = None
+        # positions from which a step's attention is split over the keys: such steps replay graphs of their own
+        self.keys_from = ops.attention_keys_from(B, tm.cfg.H, tm.cfg.KV, tm.cfg.hd, tm.Smax)
+        self.graph, self.graphs = None, {}   # the last captured step; (split over the keys, trace buffer) -> captured step
         self.trace = trace
         self.nstep = 0
         self.recorder = None
         if trace:
             self.layout = TraceLayout(tm.w, B)
             self.trace_bufs = [torch.zeros(self.layout.total, dtype=I64, device=tm.dev) for _ in range(2)]
-            self.graphs = [None, None]
 
     def record(self, mode="commit", keep=False):
         """Attach a TraceRecorder (modes "device", "host", "commit"); returns it."""
@@ -832,31 +849,43 @@ class GraphDecoder:
         ws.slot.copy_(torch.arange(self.B, dtype=I32))
         ws.pos.copy_(torch.tensor(self.cache.n[:self.B], dtype=I32))
 
-    def _step(self, b=0):
+    def _split(self):
+        """whether the next step's attention is split over the keys"""
+        return max(self.cache.n[:self.B]) + 1 >= self.keys_from
+
+    def _step(self, b=0, split=None):
         self.tm._cache = self.cache
-        self.tm.forward_rows(self.ws, trace=(self.layout, self.trace_bufs[b]) if self.trace else None, independent=True)
+        split = self._split() if split is None else split
+        self.tm.forward_rows(self.ws, trace=(self.layout, self.trace_bufs[b]) if self.trace else None, independent=True,
+                             keys=self.tm.Smax if split else 1)
         ops.advance(self.ws.pos)
 
     def capture(self):
-        """Warm up once outside the graph (restoring positions), then capture one step (one per trace buffer)."""
+        """Warm up once outside the graph (restoring positions), then capture one step (one per trace buffer, and one more
+        each for the attention split over the keys where the positions can still grow into it)."""
         ws = self.ws
         pos0 = ws.pos.clone()
         ids0 = ws.ids.clone()
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
+        modes = [True] if self._split() else [False] + [True] * (self.keys_from <= self.tm.Smax)
+        if True in modes:
+            self.tm.attention_work(ws)   # on this stream, as the workspace's other buffers
         with torch.cuda.stream(s):
-            self._step()
+            for m in modes:
+                self._step(split=m)
+                ws.pos.copy_(pos0)
+                ws.ids.copy_(ids0)
         torch.cuda.current_stream().wait_stream(s)
         ws.pos.copy_(pos0)
         ws.ids.copy_(ids0)
         torch.cuda.synchronize()
-        for b in range(2 if self.trace else 1):
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
-                self._step(b)
-            if self.trace:
-                self.graphs[b] = g
-            self.graph = g
+        for m in modes:
+            for b in range(2 if self.trace else 1):
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g):
+                    self._step(b, m)
+                self.graph = self.graphs[m, b] = g
         torch.cuda.synchronize()
 
     def step(self):
@@ -869,12 +898,11 @@ class GraphDecoder:
         b = self.nstep % 2
         if self.recorder is not None:
             self.recorder.before_step(b)
-        if self.graph is None:
+        if not self.graphs:
             self._step(b)
-        elif self.trace:
-            self.graphs[b].replay()
         else:
-            self.graph.replay()
+            split = self._split() or (False, 0) not in self.graphs   # the same results from either
+            self.graphs[split, b if self.trace else 0].replay()
         if self.recorder is not None:
             self.recorder.after_step(b)
         self.nstep += 1

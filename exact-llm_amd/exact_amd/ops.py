@@ -454,10 +454,39 @@ def attention(qq, sq, cache, slot, pos, expt, out, H, KV, hd, inv, obits=None):
 ATT_SPLIT_MAX = 4   # bit lengths a head that attention_qkv may write (blocks a head's p.V may take)
 
 
-def attention_qkv(t, s, b, cos_t, sin_t, slot, pos, cache, expt, out, H, KV, hd, inv, obits=None, obn=1):
-    """qkv_rope_cache + attention in one launch for rows that each own their (slot, position); t unchanged.
+# Decode attention split over the keys (exact_attention_decode, four launches) against one launch with a block per (row,
+# head), whose time grows with the positions: in a graph, us a layer at 17 / 301 / 601 / 6002 positions, one row of 28 heads
+# over 4 KV heads of 128: 8.0 / 15.3 / 24.2 / 182 in one launch, 15.2 / 16.3 / 17.2 / 21.4 split. Heads of 64 halve the slope
+# (401 positions: 10.3 and 13.5), and caches of at most 512 positions have faster one-launch variants (401 positions of 512:
+# 11.3 and 16.1). Where the (row, head) blocks run in several rounds (8 rows of 40 heads over 8) the lines meet earlier:
+# 16.8 in two launches and 18.0 split at 131 positions, 239 and 67 at 3001.
+ATT_KEYS_WORK = 384 * 128
+ATT_KEYS_WORK_ROUNDS = 192 * 128
+ATT_ROUND_BLOCKS = 256
+ATT_SHORT_CACHE = 512
+
+
+def attention_keys_from(R, H, KV, hd, Smax):
+    """The number of positions (keys of the longest row) from which decode attention goes split over the keys; beyond Smax
+    where the split does not take the sizes."""
+    if _lib.load().exact_attention_decode_workspace(R, H, KV, hd, Smax) <= 0:
+        return Smax + 1
+    if R * H <= ATT_ROUND_BLOCKS and Smax <= ATT_SHORT_CACHE:
+        return Smax + 1
+    return (ATT_KEYS_WORK if R * H <= ATT_ROUND_BLOCKS else ATT_KEYS_WORK_ROUNDS) // hd + 1
+
+
+def attention_work(R, H, KV, hd, Smax, device):
+    """Workspace of one split attention_qkv call of these sizes."""
+    return torch.empty(max(1, int(_lib.load().exact_attention_decode_workspace(R, H, KV, hd, Smax))), dtype=I8, device=device)
+
+
+def attention_qkv(t, s, b, cos_t, sin_t, slot, pos, cache, expt, out, H, KV, hd, inv, obits=None, obn=1, keys=None, work=None):
+    """qkv_rope_cache + attention for rows that each own their (slot, position); t unchanged.
     obits (optional) gets obn entries per head (1, 2 or ATT_SPLIT_MAX; their max is the head's bit length): with obn > 1
-    the library may split each head's p.V over obn blocks, one output slice each."""
+    the library may split each head's p.V over obn blocks, one output slice each. keys: the longest row's positions when
+    the caller knows them (else the cache's): from attention_keys_from() on the call is split over the keys (work: its
+    attention_work(), else allocated here), and one launch below. The results are the same either way."""
     R = t.shape[0]
     kq, sk, v = cache
     _need(t, I64, "t", R * (H + 2 * KV) * hd)
@@ -466,10 +495,15 @@ def attention_qkv(t, s, b, cos_t, sin_t, slot, pos, cache, expt, out, H, KV, hd,
         _need(obits, I32, "obits", R * H * obn)
     args = (_ptr(t), _ptr(_need(s, I32, "s", R)), _ptr(b), _ptr(cos_t), _ptr(sin_t), _ptr(slot), _ptr(pos), _ptr(kq),
             _ptr(sk), _ptr(v), _ptr(expt), _ptr(out), _ptr(obits))
-    if obn == 1:
-        _lib.call("exact_attention_qkv", *args, R, H, KV, hd, kq.shape[2], inv, _stream())
+    Smax = kq.shape[2]
+    if min(keys or Smax, Smax) >= attention_keys_from(R, H, KV, hd, Smax) and expt.data_ptr() % 16 == 0:
+        work = attention_work(R, H, KV, hd, Smax, t.device) if work is None else work
+        _lib.call("exact_attention_decode", *args, obn, _ptr(_need(work, I8, "work")), work.numel(), R, H, KV, hd, Smax, inv,
+                  _stream())
+    elif obn == 1:
+        _lib.call("exact_attention_qkv", *args, R, H, KV, hd, Smax, inv, _stream())
     else:
-        _lib.call("exact_attention_qkv_split", *args, obn, R, H, KV, hd, kq.shape[2], inv, _stream())
+        _lib.call("exact_attention_qkv_split", *args, obn, R, H, KV, hd, Smax, inv, _stream())
     return out
 
 

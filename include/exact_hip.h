@@ -291,6 +291,19 @@ int exact_attention_qkv_split(const int64_t* t, const int32_t* s, const int64_t*
                               int64_t* v, const int32_t* exp_t, int64_t* out, int32_t* obits, int32_t obn, int32_t R,
                               int32_t H, int32_t KV, int32_t hd, int32_t Smax, int32_t INV, void* stream);
 
+/* exact_attention_qkv_split for long caches, as four launches split over the keys (scores, exponentials, p.V, output), so
+ * that one row's attention takes more CUs than it has heads and each group of H / KV query heads reads its keys and values
+ * once. Same results, cache contents and obits contract. hd 64 or 128,
+ * H / KV one of 1, 2, 4, 5, 7, 8, Smax <= 8192 (otherwise EXACT_E_UNSUPPORTED). work: device memory of at least
+ * exact_attention_decode_workspace(R, H, KV, hd, Smax) bytes (0: sizes the entry point refuses), 256-byte aligned,
+ * of this call alone while it runs. Replaces the same steps as exact_attention_qkv (exact_llm.py:170-176). */
+int64_t exact_attention_decode_workspace(int32_t R, int32_t H, int32_t KV, int32_t hd, int32_t Smax);
+int exact_attention_decode(const int64_t* t, const int32_t* s, const int64_t* b, const int64_t* cos_t,
+                           const int64_t* sin_t, const int32_t* slot, const int32_t* pos, int16_t* kq, int32_t* sk,
+                           int64_t* v, const int32_t* exp_t, int64_t* out, int32_t* obits, int32_t obn, void* work,
+                           int64_t work_bytes, int32_t R, int32_t H, int32_t KV, int32_t hd, int32_t Smax, int32_t INV,
+                           void* stream);
+
 /* The same attention for the prefill of one sequence on the matrix cores: R query rows of cache slot `slot`
  * at increasing positions pos[r] (< nkeys), against keys 0..pos[r]; results identical to exact_attention
  * (exact_llm.py:170-176; exact_torch.py:162-166). q.k runs on int8 digit products of the int16 q and k

@@ -1,20 +1,118 @@
-"""Batched decode attention of a KV head with eight query heads, against the two launches exact_qkv_rope_cache +
-exact_attention, which the oracle pins."""
+"""Decode attention split over the keys (exact_attention_decode) against the two launches exact_qkv_rope_cache +
+exact_attention, which the oracle pins: every output, cache entry and bit length equal."""
 import numpy as np
 import pytest
 import torch
 
 import exact_oracle as O
-from exact_amd import ops
+from exact_amd import ops, synth
 from exact_amd.tables import exp_t, host_tables
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
-I16, I32, I64 = torch.int16, torch.int32, torch.int64
+I8, I16, I32, I64 = torch.int8, torch.int16, torch.int32, torch.int64
 
 
 def dev(a, dt):
     return torch.tensor(np.ascontiguousarray(a), dtype=dt, device=DEV)
+
+
+def compare(H, KV, hd, Smax, pos, seed, vmag=29, table=None, obn=4, bias=True):
+    """both paths on random caches (int16 keys over their whole range) with the rows at pos, in permuted slots"""
+    rng = np.random.default_rng(seed)
+    R, N = len(pos), (H + 2 * KV) * hd
+    B = R + 1
+    kq = rng.integers(-32767, 32768, (B, KV, Smax, hd))
+    sk = rng.integers(0, 4, (B, KV, Smax))
+    v = rng.integers(-(1 << vmag), 1 << vmag, (B, KV, Smax, hd))
+    t = dev(rng.integers(-(1 << 44), 1 << 44, (R, N)), I64)
+    s = dev(rng.integers(0, 12, R), I32)
+    b = dev(rng.integers(-(1 << 20), 1 << 20, N), I64) if bias else None
+    slot, pos = dev(rng.permutation(B)[:R], I32), dev(pos, I32)
+    tabs = host_tables(Smax, hd, 1e6)
+    cos, sin, expt = dev(tabs["cos"], I64), dev(tabs["sin"], I64), dev(exp_t() if table is None else table, I32)
+    c_a = (dev(kq, I16), dev(sk, I32), dev(v, I64))
+    c_b = tuple(x.clone() for x in c_a)
+    qq, sq = torch.empty((R, H * hd), dtype=I16, device=DEV), torch.empty((R, H), dtype=I32, device=DEV)
+    out_a, out_b = (torch.full((R, H * hd), x, dtype=I64, device=DEV) for x in (-7, -9))
+    ob_a, ob_b = torch.full((R, H), -1, dtype=I32, device=DEV), torch.full((R, H, obn), -2, dtype=I32, device=DEV)
+    inv, t0 = O.inv_sqrt_hd(hd), t.clone()
+    ops.qkv_rope_cache(t, s, b, cos, sin, slot, pos, c_a, qq, sq, H, KV, hd)
+    ops.attention(qq, sq, c_a, slot, pos, expt, out_a, H, KV, hd, inv, ob_a)
+    work = ops.attention_work(R, H, KV, hd, Smax, DEV).fill_(0x5A)   # holds anything on entry
+    ops._lib.call("exact_attention_decode", *(ops._ptr(x) for x in (t, s, b, cos, sin, slot, pos, *c_b, expt, out_b, ob_b)), obn,
+                  ops._ptr(work), work.numel(), R, H, KV, hd, Smax, inv, ops._stream())
+    assert torch.equal(out_b, out_a)
+    assert torch.equal(ob_b.max(-1)[0], ob_a)
+    assert all(torch.equal(x, y) for x, y in zip(c_b, c_a))
+    assert torch.equal(t, t0)
+    return out_a
+
+
+# chunks of 128 keys: the first and last position of one, of the cache, and a cache of no whole chunks
+@pytest.mark.parametrize("H,KV,hd,Smax,pos", [
+    (7, 1, 128, 400, [0, 1, 127, 128, 129, 255, 256, 399]), (14, 2, 64, 129, [128, 127, 0]), (8, 1, 128, 1000, [999, 640]),
+    (8, 1, 64, 300, [299, 3]), (10, 2, 128, 640, [639, 511, 512]), (4, 1, 128, 200, [130]), (4, 2, 64, 257, [256, 100]),
+    (3, 3, 128, 300, [299, 127, 0]), (2, 2, 64, 8192, [8191, 8064]), (7, 1, 128, 8192, [8191])])
+@pytest.mark.parametrize("obn", [1, 4])
+def test_split_matches_two_launches(H, KV, hd, Smax, pos, obn):
+    compare(H, KV, hd, Smax, pos, H * Smax + hd, obn=obn, bias=obn == 4)
+
+
+def test_split_extreme_values_and_tables():
+    """values of more than 31 bits take 64-bit products; a table with negative entries gives p outside [0, 2^31), a table of
+    zeros gives 0"""
+    compare(7, 1, 128, 300, [299, 130], 3, vmag=62)
+    T = exp_t().copy()
+    T[1:40] = -T[1:40] // 3
+    compare(7, 1, 128, 300, [299, 130], 4, table=T)
+    T = exp_t().copy()
+    T[2:] = -(T[0] // 300)
+    compare(4, 1, 64, 600, [599, 290], 5, table=T, vmag=40)
+    assert not compare(4, 2, 128, 200, [199], 6, table=np.zeros_like(exp_t())).any()
+
+
+def test_split_positions_outside_the_cache_give_zeros():
+    H, KV, hd, Smax = 4, 2, 64, 256
+    z = lambda *sh, dt=I64: torch.zeros(sh, dtype=dt, device=DEV)
+    cache = (z(2, KV, Smax, hd, dt=I16), z(2, KV, Smax, dt=I32), z(2, KV, Smax, hd))
+    out, ob = torch.full((2, H * hd), -1, dtype=I64, device=DEV), torch.full((2, H, 4), -1, dtype=I32, device=DEV)
+    t = torch.full((2, (H + 2 * KV) * hd), 1 << 40, dtype=I64, device=DEV)
+    ops.attention_qkv(t, z(2, dt=I32), None, z(Smax, hd), z(Smax, hd), dev([0, 1], I32), dev([-1, Smax], I32), cache,
+                      dev(exp_t(), I32), out, H, KV, hd, O.inv_sqrt_hd(hd), ob, obn=4, keys=Smax,
+                      work=ops.attention_work(2, H, KV, hd, Smax, DEV))
+    ops._lib.call("exact_attention_decode", *(ops._ptr(x) for x in (t, z(2, dt=I32), None, z(Smax, hd), z(Smax, hd),
+                  dev([0, 1], I32), dev([-1, Smax], I32), *cache, dev(exp_t(), I32), out, ob)), 4,
+                  ops._ptr(ops.attention_work(2, H, KV, hd, Smax, DEV)), 1 << 30, 2, H, KV, hd, Smax, 1, ops._stream())
+    assert not out.any() and not ob.any() and not any(x.any() for x in cache)
+
+
+@pytest.mark.parametrize("B", [1, 3])
+def test_graph_decode_crosses_into_the_split(B, monkeypatch):
+    """Steps over the position from which attention is split (their graphs differ) give the same tokens and logits as the
+    one-launch attention throughout."""
+    from exact_amd.model import DeviceWeights, GraphDecoder, TModel
+    cfg = synth.CONFIGS["tiny-hd128"]
+    got = []
+    for work in (50 * 128, 1 << 30):
+        monkeypatch.setattr(ops, "ATT_KEYS_WORK", work)
+        tm = TModel(DeviceWeights.synthetic(cfg, 3, DEV), Smax=96, batch=B)
+        cache = tm.new_cache()
+        for b in range(B):
+            tm.forward([(7 * i + b) % cfg.V for i in range(47 - b)], cache, last_only=True, slot=b)
+        gd = GraphDecoder(tm, cache, B)
+        gd.load([5 + b for b in range(B)])
+        gd.capture()
+        assert len(gd.graphs) == (2 if work < 1 << 30 else 1)
+        rows = []
+        for _ in range(8):
+            lg, ids = gd.step()
+            rows.append((lg.clone(), ids.clone()))
+        got.append(rows)
+        lg, _ = tm.decode_rows(rows[-1][1].tolist(), cache)   # eager, past the line
+        rows.append((lg, lg))
+    for (a, i), (b, j) in zip(*got):
+        assert torch.equal(a, b) and torch.equal(i, j)
 
 
 def test_grouped_batch_attention_of_eight_heads():
@@ -33,5 +131,5 @@ def test_grouped_batch_attention_of_eight_heads():
     inv = O.inv_sqrt_hd(hd)
     ops.qkv_rope_cache(t, s, None, cos, sin, slot, pos, c_a, qq, sq, H, KV, hd)
     ops.attention(qq, sq, c_a, slot, pos, expt, out_a, H, KV, hd, inv)
-    ops.attention_qkv(t, s, None, cos, sin, slot, pos, c_b, expt, out_b, H, KV, hd, inv, obn=4)
+    ops.attention_qkv(t, s, None, cos, sin, slot, pos, c_b, expt, out_b, H, KV, hd, inv, obn=4, keys=1)
     assert torch.equal(out_a, out_b) and all(torch.equal(x, y) for x, y in zip(c_a, c_b))
