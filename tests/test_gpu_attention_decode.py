@@ -95,6 +95,7 @@ def test_graph_decode_crosses_into_the_split(B, monkeypatch):
     cfg = synth.CONFIGS["tiny-hd128"]
     got = []
     for work in (50 * 128, 1 << 30):
+        monkeypatch.setattr(ops, "ATT_SHORT_CACHE", 0)
         monkeypatch.setattr(ops, "ATT_KEYS_WORK", work)
         tm = TModel(DeviceWeights.synthetic(cfg, 3, DEV), Smax=96, batch=B)
         cache = tm.new_cache()
