@@ -56,6 +56,7 @@ SIGNATURES = {
     "exact_advance": [P, I32, P],
     "exact_zero": [P, I64, P],
     "exact_sample": [P, I32, I32, U64, P, I64, P, P, P, P],
+    "exact_sample_split": [P, I32, I32, U64, P, I64, P, P, P, P, I64, P],
     "exact_router_topk": [P, I32, P, P, P, P, I32, P, P, I32, I32, I32, I32, P],
     "exact_moe_dispatch": [P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, P],
     "exact_moe_route": [P, I32, P, P, P, P, I32, P, P, I32, I32, I32, I32, P, P, P, P, P, P, P, I32, P],
@@ -70,6 +71,7 @@ SIGNATURES = {
 }
 OTHER = {"exact_version": ([], ctypes.c_int), "exact_last_error": ([], ctypes.c_char_p),
          "exact_attention_decode_workspace": ([I32, I32, I32, I32, I32], ctypes.c_int64),
+         "exact_sample_workspace": ([I32, I32], ctypes.c_int64),
          "exact_attention_prefill_workspace": ([I32, I32, I32, I32, I32], ctypes.c_int64)}
 ERRORS = {1: "bad argument", 2: "unsupported size", 3: "HIP launch error"}
 

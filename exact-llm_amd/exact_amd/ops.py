@@ -559,11 +559,23 @@ def temp_num(temp):
     return int(round((1 << 16) / temp))
 
 
+# From this many logits a row is split over blocks (four launches); below, one block a row walks it (one launch). us a call at
+# 4096 / 6000 / 8192 / 16384 / 151936 logits, one row: 13.5 / 17.7 / 21.8 / 38.3 / 310 in one launch; 19.1 / 18.9 / 19.1 /
+# 19.1 / 17.9 split (bound by the host's four launches; 14.7 / 15.0 / 15.0 / 15.2 / 15.7 in a graph). Eight rows of 151936:
+# 311 and 20.6.
+SAMPLE_SPLIT_FROM = 6144
+
+
 def sample(lg, seed, step, tnum, expt, ids, p_out=None):
     """ids[r] = sample_int(lg[r], seed, step[r], tnum) (exact_llm.py:256-259), on the device."""
     R, V = lg.shape
-    _lib.call("exact_sample", _ptr(_need(lg, I64, "lg")), R, V, ctypes.c_uint64(seed), _ptr(_need(step, I32, "step", R)), tnum,
-              _ptr(expt), _ptr(_need(ids, I32, "ids", R)), _ptr(p_out), _stream())
+    args = (_ptr(_need(lg, I64, "lg")), R, V, ctypes.c_uint64(seed), _ptr(_need(step, I32, "step", R)), tnum, _ptr(expt),
+            _ptr(_need(ids, I32, "ids", R)), _ptr(p_out))
+    if V >= SAMPLE_SPLIT_FROM:
+        work = torch.empty(_lib.load().exact_sample_workspace(R, V), dtype=I8, device=lg.device)
+        _lib.call("exact_sample_split", *args, _ptr(work), work.numel(), _stream())
+    else:
+        _lib.call("exact_sample", *args, _stream())
     return ids
 
 

@@ -436,6 +436,12 @@ int exact_logits_argmax_noalloc(int64_t* t, const int32_t* s, int64_t* lg, int32
 int exact_sample(const int64_t* lg, int32_t R, int32_t V, uint64_t seed, const int32_t* step, int64_t tnum,
                  const int32_t* exp_t, int32_t* ids, int64_t* p_out, void* stream);
 
+/* exact_sample for rows of many logits, as four launches that split each row over blocks. Same results. work: device
+ * memory of at least exact_sample_workspace(R, V) bytes, 8-byte aligned, of this call alone while it runs. */
+int64_t exact_sample_workspace(int32_t R, int32_t V);
+int exact_sample_split(const int64_t* lg, int32_t R, int32_t V, uint64_t seed, const int32_t* step, int64_t tnum,
+                       const int32_t* exp_t, int32_t* ids, int64_t* p_out, void* work, int64_t work_bytes, void* stream);
+
 /* pos[r] += 1 for r < R (advances a decode step inside a captured graph; GraphDecoder.step :645). */
 int exact_advance(int32_t* pos, int32_t R, void* stream);
 

@@ -5,7 +5,7 @@ import torch
 
 import exact_oracle as O
 import helpers
-from exact_amd import ops, synth
+from exact_amd import _lib, ops, synth
 from exact_amd.model import DeviceWeights, TModel, generate, verify
 from exact_amd.tables import exp_t
 
@@ -71,3 +71,50 @@ def test_short_generations_match_oracle(n):
     orec, ogreedy, _ = O.generate(om, prompt, n, seed=7, temp=0.9)
     assert rec["tokens"] == orec["tokens"] and rec["chain"] == orec["chain"] and greedy == ogreedy
     assert verify(tm, rec) == (True, None)
+
+
+@pytest.mark.parametrize("R,V", [(1, 1), (3, 63), (2, 1023), (2, 1024), (3, 1025), (1, 6143), (2, 6144), (9, 6145), (1, 152064)])
+@pytest.mark.parametrize("temp", [0.05, 1.0])
+def test_split_rows_match_oracle(R, V, temp):
+    """exact_sample_split at the edges of its chunks, and where ops.sample changes to it; ids over the steps' own array"""
+    rng = np.random.default_rng(V * 7 + R)
+    lg = rng.integers(-(6 << 16), 6 << 16, (R, V))
+    lg[0, -1] = 9 << 16                                 # the last logit of a row is likely drawn
+    lgd, seed, tnum = torch.tensor(lg, device=DEV), 77, ops.temp_num(temp)
+    ids = torch.arange(R, dtype=I32, device=DEV) * 5 + 2
+    pd = torch.zeros((R, V), dtype=I64, device=DEV)
+    expt = torch.tensor(exp_t(), dtype=I32, device=DEV)
+    nb = _lib.load().exact_sample_workspace(R, V)
+    work = torch.full((nb,), 0x55, dtype=torch.int8, device=DEV)
+    p = lambda t: t.data_ptr()
+    _lib.call("exact_sample_split", p(lgd), R, V, seed, p(ids), tnum, p(expt), p(ids), p(pd), p(work), nb,
+              torch.cuda.current_stream().cuda_stream)
+    other = torch.zeros(R, dtype=I32, device=DEV)
+    ops.sample(lgd, seed, torch.arange(R, dtype=I32, device=DEV) * 5 + 2, tnum, expt, other)
+    got, gp = host(ids), host(pd)
+    for r in range(R):
+        tok, pr = O.sample_int(lg[r], seed, 5 * r + 2, tnum)
+        assert np.array_equal(gp[r], pr), r
+        assert got[r] == tok == int(other[r]), (r, got[r], tok)
+
+
+def test_split_rows_of_a_table_with_negative_entries_match_the_one_block_kernel():
+    """prefix sums that decrease: both entry points count the sums up to the target alike"""
+    V, R, seed, tnum = 5000, 3, 11, ops.temp_num(1.0)
+    rng = np.random.default_rng(4)
+    tab = np.array(exp_t(), dtype=np.int64)
+    tab[700:1500] = -(tab[700:1500] // 3)
+    expt = torch.tensor(tab, dtype=I32, device=DEV)
+    lg = torch.tensor(rng.integers(-(3 << 16), 3 << 16, (R, V)), device=DEV)
+    step = torch.arange(R, dtype=I32, device=DEV)
+    out = []
+    for lim in (V + 1, 1):
+        ids, pd = torch.zeros(R, dtype=I32, device=DEV), torch.zeros((R, V), dtype=I64, device=DEV)
+        old, ops.SAMPLE_SPLIT_FROM = ops.SAMPLE_SPLIT_FROM, lim
+        try:
+            ops.sample(lg, seed, step, tnum, expt, ids, pd)
+        finally:
+            ops.SAMPLE_SPLIT_FROM = old
+        out.append((host(ids), host(pd)))
+    assert (out[0][1] < 0).any()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
