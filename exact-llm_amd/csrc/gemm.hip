@@ -667,6 +667,27 @@ __global__ __launch_bounds__(256) void k_gather_rows_a8(const int8_t* __restrict
   }
 }
 
+// K splits of a GEMM on the A8 kernel: blocks that walk fewer groups each, against every split adding its own R x N 64-bit
+// totals. us by group walked and by 10^6 atomic adds, from sweeps over 14 shapes of N 896..37888 and K 896..18944 at 17 to
+// 253 output rows: 0.8 in 128-row tiles, 0.52 in 256-row tiles, and 4.7. Never more blocks than CUs (a split just past one
+// block a CU is slower than the one before: 40 column tiles at 41 rows 15.3 us in 6 splits, 17.8 in 7). Powers of two that
+// kept 8 groups a block, used before: 4608 x 3584 at 41 rows 16.9 us (2 splits), now 12.5 (5); 2048 x 2048 at 41 rows 10.6
+// and 7.4; 6144 x 2048 at 253 rows 27.6 (2) and 20.9 (none: the split cost more than it gave).
+static int gemm_ksplit(int tiles, int G, int64_t rows, int64_t N, bool tiles128, bool zeroed) {
+  const double group = tiles128 ? 0.8 : 0.52, add = 4.7e-6 * (double)rows * (double)N;
+  const double clear = zeroed ? 0.0 : 1.2 + (double)rows * (double)N * 8 / 4e6;   // t's zero fill: one more launch
+  int best = 1;
+  double cost = group * G + add;
+  for (int k = 2; k <= G && (int64_t)tiles * k <= 256; ++k) {
+    const double c = group * ((G + k - 1) / k) + add * k + clear;
+    if (c < cost) {
+      cost = c;
+      best = k;
+    }
+  }
+  return best;
+}
+
 template <int ABITS, int WM, int WN, int S>
 static int gemm_launch(const void* x, const int8_t* wp, const int16_t* mp, int64_t* t, int M, int N, int K,
                        hipStream_t st, int ksplit_req, bool zeroed = false) {
@@ -753,10 +774,7 @@ static int gemm_launch_a8p_t(const void* x, const int8_t* wp, const int16_t* mp,
   const int G = K / 128, nbs = (N + 63) / 64;
   const int tiles_m = (M + C::BM - 1) / C::BM, tiles_n = (nbs + C::NT - 1) / C::NT;
   int ksplit = ksplit_req;
-  if (ksplit <= 0) {
-    ksplit = 1;
-    while (tiles_m * tiles_n * ksplit < GEMM_SPLIT_TILES && G / (ksplit * 2) >= 8) ksplit *= 2;
-  }
+  if (ksplit <= 0) ksplit = gemm_ksplit(tiles_m * tiles_n, G, PAIRS ? M / 2 : M, N, WM == 2, zeroed);
   if (ksplit > G) ksplit = G;
   // one K pass over enough tiles: the assembly main loop (same tiles and outputs; 32-bit offsets into x, W and t)
   if (GEMM_ASM && ksplit == 1 && !WIDE && WM == 4 && WN == 2 &&

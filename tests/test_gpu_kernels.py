@@ -72,6 +72,22 @@ def test_gemm_rows(thr, abits, R):
     assert np.array_equal(host(t), oracle_t(xq, synth.weights_np(kw, N, K), synth.scales_np(km, N, K)))
 
 
+@pytest.mark.parametrize("abits", [15, 7])
+@pytest.mark.parametrize("R,N,K", [(17, 61, 2048), (19, 130, 128), (33, 200, 896), (64, 1152, 896), (65, 1152, 1664),
+                                   (129, 328, 4864), (253, 64, 1408)])
+def test_gemm_k_splits(thr, abits, R, N, K):
+    """K splits of uneven length (1 to 38 of them, in both tile sizes), whole output, into a cleared and an uncleared t"""
+    lin, kw, km = synth_lin(thr, 33, "split", N, K)
+    lim = (1 << abits) - 1
+    xq = rng.integers(-lim, lim + 1, (R, K))
+    x = dev(xq, I16 if abits == 15 else I8)
+    exp = oracle_t(xq, synth.weights_np(kw, N, K), synth.scales_np(km, N, K))
+    t = torch.full((R, N), 7, dtype=I64, device=DEV)
+    assert np.array_equal(host(ops.gemm_g128(x, abits, lin, t)), exp)
+    t.zero_()
+    assert np.array_equal(host(ops.gemm_g128(x, abits, lin, t, zeroed=True)), exp)
+
+
 @pytest.mark.parametrize("name,N,K", [("gateup", 18944, 3584), ("down", 3584, 18944)])
 def test_prefill_gemm_full_shapes(thr, name, N, K):
     """The 2048-token prefill GEMMs at full size, A8 (the benchmark) and A16 (the spec): 40 whole output rows and
