@@ -776,6 +776,7 @@ static int gemm_launch_a8p_t(const void* x, const int8_t* wp, const int16_t* mp,
   int ksplit = ksplit_req;
   if (ksplit <= 0) ksplit = gemm_ksplit(tiles_m * tiles_n, G, PAIRS ? M / 2 : M, N, WM == 2, zeroed);
   if (ksplit > G) ksplit = G;
+  // (exact_gemm_g128_splits repeats this choice)
   // one K pass over enough tiles: the assembly main loop (same tiles and outputs; 32-bit offsets into x, W and t)
   if (GEMM_ASM && ksplit == 1 && !WIDE && WM == 4 && WN == 2 &&
       (int64_t)(PAIRS ? M / 2 : M) * N * 8 < (1LL << 32) && (int64_t)G * nbs * 8192 < (1LL << 32))
@@ -940,4 +941,13 @@ extern "C" int exact_gemm_g128_digits(const int8_t* x8, const int8_t* wp, const 
   if (2 * (int64_t)R * K >= (1LL << 32)) return EXACT_E_UNSUPPORTED;   // 32-bit buffer offsets of the digit rows
   return gemm_launch_a8p<GEMM_A8P_CFG, true>(x8, wp, mp, mh, t, 2 * R, N, K, as_stream(stream), GEMM_KSPLIT, colterm,
                                              zeroed != 0);
+}
+
+extern "C" int exact_gemm_g128_splits(int32_t abits, int32_t R, int32_t N, int32_t K) {
+  const int64_t M = (abits == 15 ? 2 : 1) * (int64_t)R;
+  if ((abits != 15 && abits != 7) || R <= 16 || N <= 0 || K <= 0 || K % 128 || M * K >= (1LL << 32)) return 0;
+  if (GEMM_KSPLIT > 0) return GEMM_KSPLIT;
+  const int64_t tiles_m = cdiv(M, M <= GEMM_SMALL_M ? 128 : 256), tiles_n = cdiv(cdiv(N, 64), 2);
+  if (tiles_m * tiles_n > 256) return 1;
+  return gemm_ksplit((int)(tiles_m * tiles_n), K / 128, R, N, M <= GEMM_SMALL_M, true);
 }

@@ -264,7 +264,7 @@ class TModel:
         self.nl = len(weights.layers)
         self.nq = (c.H + 2 * c.KV) * c.hd
         self.I = c.I if not c.moe else 1
-        self._ws = {}
+        self._ws, self._adds_R = {}, {}
         self._pws = None
         self._graphs = collections.OrderedDict()   # captured prefill passes
 
@@ -321,6 +321,14 @@ class TModel:
         ops.requant_channel(acc, s, lin.M, lin.Mbits, lin.bias, out=out)
         return out
 
+    def _adds(self, R):
+        """{linear of a layer: whether its call on R rows may add into its totals} (ops.linear_adds)"""
+        if R not in self._adds_R:
+            L = self.w.layers[0]
+            self._adds_R[R] = {n: ops.linear_adds(R, self.abits, L[n]) for n in ("qkv", "o", "gateup", "down", "router",
+                                                                               "sgu", "sd") if n in L}
+        return self._adds_R[R]
+
     # ---------------------------------------------------------------- one pass over R rows
     def forward_rows(self, ws, want_logits=True, trace=None, independent=False, last_only=False, keys=None):
         """Runs the model on ws.ids with (slot, pos) per row; KV of each row is written into the cache
@@ -345,6 +353,11 @@ class TModel:
             tbuf.zero_()
             slot = lambda key: layout.slot(tbuf, key)
         clear = group and not keep
+        # which totals their consumer leaves zeroed: those that the next pass's linear adds into. The GEMMs of a prompt that
+        # split no K write theirs whole, and clearing them is as many bytes again as reading them (a layer of the 7B shape at
+        # 1537 tokens: SwiGLU launch 141 -> 120 us, its qrow 105 -> 69, q|k|v epilogue 42 -> 35, norms 42 -> 35.5 each)
+        adds = self._adds(R)
+        c_qkv, c_o, c_gu, c_d = (clear and adds.get(n, True) for n in ("qkv", "o", "gateup", "down"))
         # decode passes of up to QROW_FUSE_ROWS rows: the o and down GEMVs quantise their int64 inputs themselves (no
         # qrow launch); every 64-row block of the GEMV re-reads its slice of the row, which costs more than the saved
         # launch at 8 rows
@@ -410,7 +423,7 @@ class TModel:
                     x_cur, x_nxt = x_nxt, x_cur
                 s_qkv, b_qkv = ws.s, L["qkv"].bias
             else:
-                ops.rmsnorm_qrow(x_cur, L["g1"], self.abits, res_t, res_s, ws.xq, ws.s, clear=clear, x8=dx)
+                ops.rmsnorm_qrow(x_cur, L["g1"], self.abits, res_t, res_s, ws.xq, ws.s, clear=c_d, x8=dx)
             if nfuse or qfuse:
                 pass
             elif group:
@@ -431,7 +444,7 @@ class TModel:
                 nob = H * self.ATT_SPLIT
             else:
                 ops.qkv_rope_cache(t_qkv if group else ws.t_qkv, s_qkv, b_qkv, tab.cos, tab.sin, ws.slot, ws.pos, cache,
-                                   ws.qq, ws.sq, H, KV, hd, clear=clear)
+                                   ws.qq, ws.sq, H, KV, hd, clear=c_qkv)
                 if ws.seq is not None:
                     ops.attention_prefill(ws.qq, ws.sq, cache, ws.seq[0], ws.pos, ws.seq[1], tab.exp, ws.att, H, KV, hd,
                                           tab.inv, self._prefill_ws(R), ws.obits)
@@ -443,7 +456,7 @@ class TModel:
                 ops.gemv_qrow_acc(ws.att, ws.obits, nob, self.abits, L["o"], t_o, ws.sa,
                                   zero=(ws.t_qd if qfuse else t_qkv) if afuse and clear else None)
             else:
-                ops.quant_rows(ws.att, ws.obits, nob, self.abits, ws.aq, ws.sa, x8=da, zero=t_qkv if bfuse and clear else None)
+                ops.quant_rows(ws.att, ws.obits, nob, self.abits, ws.aq, ws.sa, x8=da, zero=t_qkv if bfuse and c_qkv else None)
             if nfuse and nsfuse:   # norm + gate|up + SwiGLU in one launch
                 ops.gemv_norm_swiglu(x_cur, t_o, ws.sa, L["g2"], L["gateup"], ws.s, tab.silu, ws.h, ws.part_sw,
                                      x_out=x_nxt, t=t_gu if keep else None)
@@ -469,7 +482,7 @@ class TModel:
                 elif fsfuse:
                     pass
                 else:
-                    ops.rmsnorm_qrow(x_cur, L["g2"], self.abits, t_o, ws.sa, ws.xq, ws.s, clear=clear, x8=dx)
+                    ops.rmsnorm_qrow(x_cur, L["g2"], self.abits, t_o, ws.sa, ws.xq, ws.s, clear=c_o, x8=dx)
             else:
                 self._lin_channel(ws.aq, ws.sa, L["o"], ws.t_o)
                 ops.rmsnorm_qrow(ws.x, L["g2"], self.abits, ws.t_o, ws.s28, ws.xq, ws.s)
@@ -501,7 +514,7 @@ class TModel:
                     ops.swiglu_part(t_gu, ws.s, tab.silu, ws.h, ws.part_sw, clear=clear)
                     ops.gemv_qrow_acc(ws.h, ws.part_sw, -(-c.I // ops.QSLICE), self.abits, L["down"], t_d, ws.sh)
                 else:
-                    ops.swiglu_qrow(t_gu, ws.s, tab.silu, self.abits, ws.hq, ws.sh, clear=clear, part=ws.part_sw,
+                    ops.swiglu_qrow(t_gu, ws.s, tab.silu, self.abits, ws.hq, ws.sh, clear=c_gu, part=ws.part_sw,
                                     h=ws.h if keep else None, x8=dh)
                     self._lin(ws.hq, L["down"], t_d, x8=dh)
                 res_t, res_s = t_d, ws.sh
@@ -525,10 +538,10 @@ class TModel:
             # a prompt's last row only: its final norm, head GEMV and argmax; the other rows' residual totals are
             # cleared for the next pass that accumulates into them
             r = slice(R - 1, R)
-            if clear and res_t is not None:
+            if c_d and res_t is not None:
                 ops.zero_(res_t[:R - 1])
             ops.rmsnorm_qrow(x_cur[r], self.w.gf, self.abits, None if res_t is None else res_t[r],
-                             None if res_s is None else res_s[r], ws.xq[r], ws.s[r], clear=clear)
+                             None if res_s is None else res_s[r], ws.xq[r], ws.s[r], clear=c_d)
             if head.mode == "group":
                 self._lin(ws.xq[r], head, ws.t_head[r])
                 ops.logits_argmax(ws.t_head[r], ws.s[r], ws.logits[r] if want_logits else None, ws.next_ids[r],
@@ -539,7 +552,7 @@ class TModel:
                 ops.logits_argmax(ws.t_head[r], ws.s28[r], ws.logits[r] if want_logits else None, ws.next_ids[r],
                                   part=ws.part_lg)
             return ws
-        ops.rmsnorm_qrow(x_cur, self.w.gf, self.abits, res_t, res_s, ws.xq, ws.s, clear=clear, x8=dx)
+        ops.rmsnorm_qrow(x_cur, self.w.gf, self.abits, res_t, res_s, ws.xq, ws.s, clear=c_d, x8=dx)
         if head.mode == "group":
             t_head = slot("head") if keep else ws.t_head
             self._lin(ws.xq, head, t_head, x8=dx)
@@ -559,6 +572,7 @@ class TModel:
         isig-gated shared expert. routed: the router totals ws.t_rt are already there (the norm-fused router GEMV);
         zero: an int64 tensor to clear on the way (the shared expert's down GEMV clears it, or a launch of its own)."""
         c, tab, k = self.cfg, self.tab, self.cfg.topk
+        adds = self._adds(ws.R)
         P = ws.R * k
         x = ws.x if x is None else x
         if not routed:
@@ -573,7 +587,7 @@ class TModel:
             ops.moe_route(ws.t_rt, ws.s, tab.exp, k, ws.p_sel, ws.e_sel, chunk, ws.disp, clear=True, NE=c.NE,
                           gate_col=ws.gate_col, sig=tab.sig, gate=ws.gate)
         else:
-            ops.router_topk(ws.t_rt, ws.s, tab.exp, k, ws.p_sel, ws.e_sel, clear=True, NE=c.NE, gate_col=ws.gate_col,
+            ops.router_topk(ws.t_rt, ws.s, tab.exp, k, ws.p_sel, ws.e_sel, clear=adds["router"], NE=c.NE, gate_col=ws.gate_col,
                             sig=tab.sig, gate=ws.gate)
             ops.moe_dispatch(ws.e_sel, ws.s, c.NE, k, chunk, ws.disp)
         sfuse = (self.SHARED_SWIGLU and not grouped and self.abits == 15 and ws.R <= ops.SWIGLU_GEMV_ROWS and c.SI % 64 == 0
@@ -614,11 +628,13 @@ class TModel:
                               zero=zero)
         else:
             self._lin(ws.xq, L["sgu"], ws.t_sgu, x8=dx)
-            ops.swiglu_qrow(ws.t_sgu, ws.s, tab.silu, self.abits, ws.shq, ws.ssh, clear=True, part=ws.part_sw, x8=dh)
+            ops.swiglu_qrow(ws.t_sgu, ws.s, tab.silu, self.abits, ws.shq, ws.ssh, clear=adds["sgu"], part=ws.part_sw, x8=dh)
             self._lin(ws.shq, L["sd"], ws.t_sd, x8=dh)
             if zero is not None:
                 ops.zero_(zero)
-        ops.moe_combine(x, ws.t_ed, ws.esh, ws.p_sel, ws.disp["pidx"], k, ws.t_sd, ws.ssh, ws.gate, clear=True)
+        # the experts' GEMM writes all of t_ed
+        ops.moe_combine(x, ws.t_ed, ws.esh, ws.p_sel, ws.disp["pidx"], k, ws.t_sd, ws.ssh, ws.gate,
+                        clear=not grouped or adds["sd"])
 
     # ---------------------------------------------------------------- reference-shaped API
     PREFILL_GRAPHS = 8   # captured prefill passes kept (least recently used dropped)

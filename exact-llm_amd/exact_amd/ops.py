@@ -297,6 +297,12 @@ def linear_t(x, abits, lin, out=None, zeroed=False, x8=None):
     return gemm_g128(x, abits, lin, out, zeroed=zeroed, x8=x8)
 
 
+def linear_adds(R, abits, lin):
+    """Whether linear_t(..., zeroed=True) of R rows (int16 rows above A16_DIGIT_ROWS: given as digit rows) may add into its
+    output, which must then hold zeros; if not, every total is written and the output may hold anything."""
+    return _lib.load().exact_gemm_g128_splits(abits, R, lin.N, lin.K) != 1
+
+
 def _need_packed(lin, fn):
     """The packed buffers of lin hold ceil(N/64) * G tiles: wp int8 8192 B, mp (and mh) int16 64 per tile."""
     if lin.K <= 0 or lin.K % 128:

@@ -117,6 +117,11 @@ int exact_gemm_g128(const void* x, int32_t abits, const int8_t* wp, const int16_
 int exact_gemm_g128_zeroed(const void* x, int32_t abits, const int8_t* wp, const int16_t* mp, const int16_t* mh,
                            int64_t* t, int32_t R, int32_t N, int32_t K, void* stream);
 
+/* The K splits exact_gemm_g128_zeroed (int8 rows) and exact_gemm_g128_digits with zeroed (int16 rows) run R > 16 rows in:
+ * with 1 they write every total without reading t, so that t need not hold zeros; with more they add into it. 0: sizes
+ * that these entries refuse or run on another path, which may add. */
+int exact_gemm_g128_splits(int32_t abits, int32_t R, int32_t N, int32_t K);
+
 /* qrow fused into the GEMV that consumes it: t += qrow(xs, abits) . W (t holds zeros or a running total), where
  * row r of xs (int64, ldx apart) is quantised with s = max(max_i part[r * nparts + i] - abits, 0) and
  * part holds the producer's bit lengths of max |xs| over slices of the row (exact_attention's per-head

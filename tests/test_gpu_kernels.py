@@ -74,9 +74,10 @@ def test_gemm_rows(thr, abits, R):
 
 @pytest.mark.parametrize("abits", [15, 7])
 @pytest.mark.parametrize("R,N,K", [(17, 61, 2048), (19, 130, 128), (33, 200, 896), (64, 1152, 896), (65, 1152, 1664),
-                                   (129, 328, 4864), (253, 64, 1408)])
+                                   (129, 328, 4864), (253, 64, 1408), (300, 1000, 256)])
 def test_gemm_k_splits(thr, abits, R, N, K):
-    """K splits of uneven length (1 to 38 of them, in both tile sizes), whole output, into a cleared and an uncleared t"""
+    """K splits of uneven length (1 to 38 of them, in both tile sizes), whole output, into a cleared and an uncleared t; where
+    linear_adds says that a linear does not add, its "zeroed" form writes every total of an uncleared t as well"""
     lin, kw, km = synth_lin(thr, 33, "split", N, K)
     lim = (1 << abits) - 1
     xq = rng.integers(-lim, lim + 1, (R, K))
@@ -86,6 +87,14 @@ def test_gemm_k_splits(thr, abits, R, N, K):
     assert np.array_equal(host(ops.gemm_g128(x, abits, lin, t)), exp)
     t.zero_()
     assert np.array_equal(host(ops.gemm_g128(x, abits, lin, t, zeroed=True)), exp)
+    if R == 300:
+        assert not ops.linear_adds(R, abits, lin)
+    if not ops.linear_adds(R, abits, lin):
+        x8 = None
+        if abits == 15:
+            x8 = dev(np.stack([xq >> 8, (xq & 255) - 128], 1).reshape(2 * R, K), I8)
+        t.fill_(7)
+        assert np.array_equal(host(ops.linear_t(x, abits, lin, t, zeroed=True, x8=x8)), exp)
 
 
 @pytest.mark.parametrize("name,N,K", [("gateup", 18944, 3584), ("down", 3584, 18944)])

@@ -229,3 +229,28 @@ def test_last_only_prefill_matches_full_prefill(name, abits, T):
     a = host(tm.forward(more, c1))
     b = host(tm.forward(more, c2, last_only=True))
     assert np.array_equal(b[0], a[-1])
+
+
+@pytest.mark.parametrize("name,abits,T", [("tiny", 15, 20), ("tiny", 15, 300), ("tiny-moe", 15, 300), ("tiny", 7, 300)])
+def test_prompts_over_stale_totals(name, abits, T):
+    """Prompts of one length in turn (whole logits, then the last row's, then whole again) against fresh models: totals that
+    a pass leaves behind do not reach the next one, whether its GEMMs add into them (short prompts) or write them whole."""
+    cfg = synth.CONFIGS[name]
+    make = lambda: TModel(DeviceWeights.synthetic(cfg, 21, "cuda"), Smax=T + 8, abits=abits)
+    tm = make()
+    if T == 300:
+        assert not all(tm._adds(T).values())
+        ws = tm.workspace(T)
+        for n, t in (("qkv", "t_qkv"), ("o", "t_o"), ("gateup", "t_gu"), ("down", "t_d"), ("sgu", "t_sgu"), ("sd", "t_sd")):
+            if not tm._adds(T).get(n, True):
+                getattr(ws, t).fill_(12345)
+    for i, last in enumerate((False, True, False, True)):
+        ids = helpers.prompt(i, T, cfg.V)
+        fresh, c0 = make(), tm.new_cache(B=1)
+        c1 = fresh.new_cache(B=1)
+        a = host(tm.forward(ids, c0, last_only=last))
+        b = host(fresh.forward(ids, c1))
+        assert np.array_equal(a, b[-1:] if last else b), (i, last)
+        assert all(torch.equal(u, v) for x, y in zip(c0.layers, c1.layers) for u, v in zip(x, y))
+        la, lb = tm.decode_rows([3], c0)[0], fresh.decode_rows([3], c1)[0]
+        assert torch.equal(la, lb)
