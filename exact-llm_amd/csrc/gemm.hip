@@ -554,16 +554,68 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void k_gemm_a8p(const int8_t* __re
 #include "../_build/gemm_asm.inc"
 namespace exact {
 
+// ---- SwiGLU in the gate|up GEMM's epilogue: h = shr(isilu(shr(g, 28 - s)) shr(u, 28 - s), 16) from the totals of a lane's two
+// gate and up columns (T(rs, jp, cs): rows orow + 8 rs + jp, columns c0 + (cs & 1), cs >= 2 the up half). A row's 32 columns of
+// a wave are one slice: its bit length of max |h| goes to part[row * I / 32 + slice], and its h to 32 int64 slots of h, as int32
+// in the first half of them when they all fit (bit length <= 31), which halves what the launch stores and the quantising one
+// reads. The totals (two int64 an output) stay in registers: a 7B layer at 1537 rows stored and read back 933 MB of them, 504 us
+// of GEMM and 120 of SwiGLU launch, now 538 (the epilogue's 8192 outputs a block run beside no other block of the CU).
+struct SwigluOut {
+  const int32_t* s;      // (R) shifts of the GEMM's rows
+  const int32_t* silu;
+  int64_t* h;
+  int32_t* part;
+};
+
+__device__ __forceinline__ int64_t silu_mul(const int32_t* T, int64_t g, int64_t u) {
+  // lut16(T, g): (b - a) fr + 128 as two 32 x 32 + 64 multiply-adds
+  const int t = ((int)g + (16 << EXACT_F)) & ((32 << EXACT_F) - 1), fr = t & 255;
+  const int a = T[t >> 8], b = T[(t >> 8) + 1];
+  int64_t y = (int64_t)a + (((int64_t)b * fr + ((int64_t)a * -fr + 128)) >> 8);
+  y = g >= (16LL << EXACT_F) ? g : (g < -(16LL << EXACT_F) ? 0 : y);
+  return (int64_t)((uint64_t)y * (uint64_t)u + (1ULL << (EXACT_F - 1))) >> EXACT_F;
+}
+
+__device__ __forceinline__ void swiglu_epilogue(const v32i& t0, const v32i& t1, int orow, int Mout, int c0, int I, int slice,
+                                                int j, const SwigluOut& sw) {
+  auto total = [&](int k) {   // int64 k of the lane's 32
+    const int lo = k < 16 ? t0[2 * k] : t1[2 * k - 32], hi = k < 16 ? t0[2 * k + 1] : t1[2 * k - 31];
+    return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+  };
+  const int np = I / 32;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {   // row orow + 8 rs + jp, k = 2 rs + jp
+    const int row = orow + 8 * (k >> 1) + (k & 1);
+    const int sh = 28 - sw.s[row < Mout ? row : Mout - 1];
+    int64_t h[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) h[c] = silu_mul(sw.silu, shr64(total(4 * k + c), sh), shr64(total(4 * k + 2 + c), sh));
+    int m = bitlen64((int64_t)((uint64_t)abs64(h[0]) | (uint64_t)abs64(h[1])));   // bitlen of the or = the larger one's
+    auto mx = [](int a, int b) { return a > b ? a : b; };
+    m = mx(m, dpp32<0xB1>(m));
+    m = mx(m, dpp32<0x4E>(m));
+    m = mx(m, dpp32<0x141>(m));
+    m = mx(m, dpp32<0x140>(m));
+    if (row < Mout) {
+      int64_t* dst = sw.h + (int64_t)row * I + (c0 - 2 * j);
+      if (m <= 31) reinterpret_cast<int2*>(dst)[j] = make_int2((int)h[0], (int)h[1]);
+      else reinterpret_cast<longlong2*>(dst)[j] = make_longlong2(h[0], h[1]);
+      if (j == 0) sw.part[(int64_t)row * np + slice] = m;
+    }
+  }
+}
+
 // The A8 GEMM (and A16 as digit-row pairs) with its main loop in generated assembly (gen_gemm_asm.py, which states
 // the schedule and the register map): 256 x 128 tiles (128 x 128 output rows x columns for PAIRS), one K pass, plain
 // stores. This function computes the block's tile, every per-lane copy / read / store offset and the scalar state,
 // and hands them to the asm in pinned registers. Mrows: rows of the A operand (digit rows for PAIRS); tiles past
 // M or N (ragged edges) store under a lane mask; A rows past Mrows read row Mrows - 1 (never stored).
-template <bool PAIRS>
+template <bool PAIRS, bool SWIGLU = false>
 __global__ __launch_bounds__(512, 1) void k_gemm_asm(const int8_t* __restrict__ xb, const int8_t* __restrict__ wp,
                                                      const int16_t* __restrict__ mp, int64_t* __restrict__ t,
                                                      const int64_t* __restrict__ colterm, int Mrows, int N, int K, int G,
-                                                     int nbs, int tiles_m, int tiles_n) {
+                                                     int nbs, int tiles_m, int tiles_n, SwigluOut sw) {
+  static_assert(PAIRS || !SWIGLU, "the SwiGLU epilogue takes int16 rows");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -574,7 +626,8 @@ __global__ __launch_bounds__(512, 1) void k_gemm_asm(const int8_t* __restrict__ 
   const int lb = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (lb >= nblk) return;
   const int bn = lb / tiles_m, bm = lb - bn * tiles_m;
-  const int row0 = bm * 256, nb0 = bn * 2, col0 = nb0 * 64;
+  const int row0 = bm * 256, nb0 = SWIGLU ? bn : bn * 2, col0 = nb0 * 64;
+  const int up = SWIGLU ? nbs / 2 : 0;   // tiles from a gate tile to its up tile
   const int g0 = 0, g1 = G;
   const int iters = __builtin_amdgcn_readfirstlane((g1 - g0 + 5) / 6);
   const int phase = __builtin_amdgcn_readfirstlane(6 * iters - (g1 - g0));
@@ -587,17 +640,20 @@ __global__ __launch_bounds__(512, 1) void k_gemm_asm(const int8_t* __restrict__ 
     const int gr = row0 + r < Mrows ? row0 + r : Mrows - 1;
     vad[i] = (uint32_t)gr * (uint32_t)K + (uint32_t)(c * 16);
   }
-  // B: LDS slot 16 cs + j of each 1 KiB chunk holds column 4 j + cs of the packed tile
-  const int vbdma = (4 * (lane & 15) + (lane >> 4)) * 16;
+  // B: LDS slot 16 cs + j of each 1 KiB chunk holds column 4 j + cs of the packed tile. SWIGLU: columns 2 j, 2 j + 1 of
+  // half wn of the gate tile (cs 0, 1) and of the up tile (cs 2, 3), so a lane has both totals of its two outputs
+  const int vbdma = SWIGLU ? (32 * (wave >> 2) + 2 * (lane & 15) + (lane >> 4 & 1)) * 16 + (lane >> 5) * up * 8192
+                           : (4 * (lane & 15) + (lane >> 4)) * 16;
   int bc[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int seg = wave * 2 + i;
-    const int tl = nb0 + (seg >> 3) < nbs ? (seg >> 3) : nbs - 1 - nb0;   // a missing second tile reads the first
+    const int tl = SWIGLU ? 0 : nb0 + (seg >> 3) < nbs ? (seg >> 3) : nbs - 1 - nb0;   // a missing second tile reads the first
     bc[i] = (nb0 + tl) * 8192 + (seg & 7) * 1024;
   }
   const int ncol = (nbs - nb0) * 64;
-  const int vmdma = (2 * lane < ncol ? 2 * lane : ncol - 2) * 2;
+  const int vmdma = SWIGLU ? (32 * (lane >> 5) + (lane & 30)) * 2 + (lane & 1) * up * 128
+                           : (2 * lane < ncol ? 2 * lane : ncol - 2) * 2;
   // LDS read bases (the asm adds stage, sub-tile and k-half offsets as immediates)
   int vard[4];
 #pragma unroll
@@ -621,15 +677,26 @@ __global__ __launch_bounds__(512, 1) void k_gemm_asm(const int8_t* __restrict__ 
   const __amdgpu_buffer_rsrc_t rT = __builtin_amdgcn_make_buffer_rsrc((void*)t, (short)0, -1, BUF_DW3);
   const int asoff = g0 * 128, bg = g0 * nbs * 8192, mg = (g0 * nbs + nb0) * 128;
   const int wavea = wave * 4096, waveb = GEMM_ASM_B_BASE + wave * 2048, wavem = GEMM_ASM_M_BASE + wave * 256;
-  if constexpr (PAIRS) {
+  if constexpr (SWIGLU) {
+    const __amdgpu_buffer_rsrc_t rCt = __builtin_amdgcn_make_buffer_rsrc((void*)colterm, (short)0, -1, BUF_DW3);
+    const int c0 = col0 + 32 * wn + 2 * j;
+    v32i t0, t1;
+    gemm_asm_main_pairs_totals(g0, g1, iters, phase, asoff, bg, bc[0], bc[1], mg, nbs * 8192, nbs * 128, wavea, waveb, wavem,
+                               N * 4, rA, rB, rM, rCt, (int)vad[0], (int)vad[1], (int)vad[2], (int)vad[3], vbdma, vmdma,
+                               vard[0], vard[1], vard[2], vard[3], vbrd, vmrd, c0 * 8, t0, t1);
+    int all = -1;
+    asm volatile("" : "+s"(all));   // the lane again from here: no VGPR is left to hold it across the main loop
+    const int ln = __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0)), lj = ln & 15;
+    swiglu_epilogue(t0, t1, row0 / 2 + wm * 32 + 2 * (ln >> 4), Mout, col0 + 32 * wn + 2 * lj, N / 2, bn * 2 + wn, lj, sw);
+  } else if constexpr (PAIRS) {
     const __amdgpu_buffer_rsrc_t rCt = __builtin_amdgcn_make_buffer_rsrc((void*)colterm, (short)0, -1, BUF_DW3);
     const int ctoff = (ocol < N ? ocol : 0) * 8;
-    gemm_asm_main_pairs(g0, g1, iters, phase, full, asoff, bg, bc[0], bc[1], mg, nbs * 8192, nbs * 128, wavea, waveb,
-                        wavem, N * 8, Mout, N, rA, rB, rM, rT, (int)vad[0], (int)vad[1], (int)vad[2], (int)vad[3], vbdma,
-                        vmdma, vard[0], vard[1], vard[2], vard[3], vbrd, vmrd, vst, orow, ocol, rCt, ctoff);
+    gemm_asm_main_pairs(g0, g1, iters, phase, asoff, bg, bc[0], bc[1], mg, nbs * 8192, nbs * 128, wavea, waveb,
+                        wavem, full, N * 8, Mout, N, rA, rB, rM, rT, rCt, (int)vad[0], (int)vad[1], (int)vad[2], (int)vad[3], vbdma,
+                        vmdma, vard[0], vard[1], vard[2], vard[3], vbrd, vmrd, vst, orow, ocol, ctoff);
   } else {
-    gemm_asm_main_a8(g0, g1, iters, phase, full, asoff, bg, bc[0], bc[1], mg, nbs * 8192, nbs * 128, wavea, waveb, wavem,
-                     N * 8, Mout, N, rA, rB, rM, rT, (int)vad[0], (int)vad[1], (int)vad[2], (int)vad[3], vbdma, vmdma,
+    gemm_asm_main_a8(g0, g1, iters, phase, asoff, bg, bc[0], bc[1], mg, nbs * 8192, nbs * 128, wavea, waveb, wavem,
+                     full, N * 8, Mout, N, rA, rB, rM, rT, (int)vad[0], (int)vad[1], (int)vad[2], (int)vad[3], vbdma, vmdma,
                      vard[0], vard[1], vard[2], vard[3], vbrd, vmrd, vst, orow, ocol);
   }
 }
@@ -754,8 +821,17 @@ static int gemm_launch_asm(const int8_t* x, const int8_t* wp, const int16_t* mp,
   const int nblk = tiles_m * tiles_n;
   const int grid = ((nblk + 7) / 8) * 8;
   hipLaunchKernelGGL(k_gemm_asm<PAIRS>, dim3(grid), dim3(512), GEMM_ASM_LDS_BYTES, st, x, wp, mp, t, colterm, M, N, K, G,
-                     nbs, tiles_m, tiles_n);
+                     nbs, tiles_m, tiles_n, SwigluOut{});
   return launch_status("gemm_g128");
+}
+
+// whether R int16 rows of a gate|up linear (2 I columns) run on the assembly main loop with the SwiGLU epilogue: the sizes on
+// which the plain GEMM splits no K and takes the assembly loop
+static bool gemm_swiglu_ok(int64_t R, int64_t I, int64_t K) {
+  if (R <= 0 || I <= 0 || K <= 0 || K % 128 || I % 64 || 2 * R <= GEMM_SMALL_M || 2 * R * K >= (1LL << 32)) return false;
+  const int64_t G = K / 128, nbs = 2 * I / 64, tiles = cdiv(2 * R, 256) * (I / 64);
+  if (!GEMM_ASM || GEMM_KSPLIT > 1 || G * nbs * 8192 >= (1LL << 32) || tiles > INT32_MAX / 2) return false;
+  return tiles > 256 || gemm_ksplit((int)tiles, (int)G, R, 2 * I, false, true) == 1;
 }
 
 // M: rows of the A operand (digit rows when PAIRS: the output has M / 2 rows, written through colterm)
@@ -950,4 +1026,27 @@ extern "C" int exact_gemm_g128_splits(int32_t abits, int32_t R, int32_t N, int32
   const int64_t tiles_m = cdiv(M, M <= GEMM_SMALL_M ? 128 : 256), tiles_n = cdiv(cdiv(N, 64), 2);
   if (tiles_m * tiles_n > 256) return 1;
   return gemm_ksplit((int)(tiles_m * tiles_n), K / 128, R, N, M <= GEMM_SMALL_M, true);
+}
+
+extern "C" int exact_gemm_swiglu_supported(int32_t R, int32_t I, int32_t K) { return gemm_swiglu_ok(R, I, K); }
+
+extern "C" int exact_gemm_g128_digits_swiglu(const int8_t* x8, const int8_t* wp, const int16_t* mp, const int64_t* colterm,
+                                             const int32_t* s, const int32_t* silu_t, int64_t* h, int32_t* part, int32_t R,
+                                             int32_t I, int32_t K, void* stream) {
+  if (!x8 || !wp || !mp || !colterm || !s || !silu_t || !h || !part || R <= 0 || I <= 0 || K <= 0) return EXACT_E_ARG;
+  if (!gemm_swiglu_ok(R, I, K) || (reinterpret_cast<uintptr_t>(x8) & 15) || (reinterpret_cast<uintptr_t>(wp) & 15) ||
+      (reinterpret_cast<uintptr_t>(h) & 15) || (reinterpret_cast<uintptr_t>(colterm) & 15))
+    return EXACT_E_UNSUPPORTED;
+  static bool attr_set = false;
+  if (!attr_set) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_asm<true, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              GEMM_ASM_LDS_BYTES);
+    attr_set = true;
+  }
+  const int tiles_m = (int)cdiv(2 * (int64_t)R, 256), tiles_n = I / 64;
+  const int64_t nblk = (int64_t)tiles_m * tiles_n;
+  hipLaunchKernelGGL((k_gemm_asm<true, true>), dim3((uint32_t)(cdiv(nblk, 8) * 8)), dim3(512), GEMM_ASM_LDS_BYTES,
+                     as_stream(stream), x8, wp, mp, nullptr, colterm, 2 * R, 2 * I, K, K / 128, 2 * I / 64, tiles_m, tiles_n,
+                     SwigluOut{s, silu_t, h, part});
+  return launch_status("gemm_g128_digits_swiglu");
 }

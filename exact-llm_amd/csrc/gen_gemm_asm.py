@@ -5,7 +5,8 @@
 
 Output: a C++ header with `gemm_asm_main_<variant>(...)`, a __device__ function whose body is a single `asm volatile`
 statement. The kernel in gemm.hip computes every per-lane and per-wave value, passes them in pinned registers, and
-calls it last; the block runs its whole K loop and stores its tile inside the asm.
+calls it last; the block runs its whole K loop and stores its tile inside the asm (the variant that ends with its totals in
+registers leaves the rest to the kernel: it serves the SwiGLU epilogue).
 
 Why assembly: the loop's matrix work (v_mfma_i32_16x16x64_i8) needs its operand fragments read from LDS well ahead
 and an exact int64 multiply-add per output per group on the vector ALUs; the compiler's schedule waits for every
@@ -324,10 +325,14 @@ def store_masked(e, pairs):
             e("s_mov_b64 exec, -1")
 
 
-def add_colterm(e):
-    """PAIRS: t += 128 * colterm[col] for the lane's four columns (loaded into the free A buffers)"""
+def add_colterm(e, totals):
+    """PAIRS: t += 128 * colterm[col] for the lane's four columns (loaded into the free A buffers). totals: columns 2, 3
+    are %[ctup] bytes past columns 0, 1"""
     e(f"buffer_load_dwordx4 {vr(V_A, 4)}, {vr(V_TMP)}, %[rCt], 0 offen")
-    e(f"buffer_load_dwordx4 {vr(V_A + 4, 4)}, {vr(V_TMP)}, %[rCt], 0 offen offset:16")
+    if totals:
+        e(f"buffer_load_dwordx4 {vr(V_A + 4, 4)}, {vr(V_TMP)}, %[rCt], %[ctup] offen")
+    else:
+        e(f"buffer_load_dwordx4 {vr(V_A + 4, 4)}, {vr(V_TMP)}, %[rCt], 0 offen offset:16")
     e("s_waitcnt vmcnt(0)")
     for cs in range(4):
         ct = V_A + 2 * cs
@@ -340,9 +345,10 @@ def add_colterm(e):
                 e(f"v_addc_co_u32 {vr(t + 1)}, vcc, {vr(t + 1)}, {vr(ct + 1)}, vcc")
 
 
-def kernel_asm(pairs):
+def kernel_asm(pairs, totals=False):
+    """totals (pairs only): end with the totals in v0..v63 instead of storing them"""
     e = Emit()
-    tag = "P" if pairs else "A"
+    tag = "T" if totals else "P" if pairs else "A"
     L = lambda n: f".Lg{tag}_{n}"
     ntot = 64 if pairs else 128
     e("s_waitcnt vmcnt(0) lgkmcnt(0)")   # nothing of the compiler's own is outstanding in the counters used below
@@ -355,7 +361,7 @@ def kernel_asm(pairs):
     e(f"v_mov_b64 {vr(V_MX + 2, 2)}, 0")
     e(f"s_mov_b32 {s('g1')}, %[g1]")
     e(f"s_mov_b32 {s('gd')}, %[g0]")
-    for nm in ("asoff", "bg", "bc0", "bc1", "mg", "nbsb", "nbsm", "wavea", "waveb", "wavem", "n8"):
+    for nm in ("asoff", "bg", "bc0", "bc1", "mg", "nbsb", "nbsm", "wavea", "waveb", "wavem") + (() if totals else ("n8",)):
         e(f"s_mov_b32 {s(nm)}, %[{nm}]")
     e(f"s_mov_b32 {s('iter')}, %[iters]")
     # entry phase k0 = 6 * iters - (g1 - g0): the first group runs as local index k0, so the last one is index 5
@@ -420,7 +426,9 @@ def kernel_asm(pairs):
     e("s_waitcnt vmcnt(0)")
     if pairs:
         e(f"v_mov_b32 {vr(V_TMP)}, %[ctoff]")
-        add_colterm(e)
+        add_colterm(e, totals)
+    if totals:
+        return e.lines
     e(f"s_cmp_eq_u32 %[full], 1")
     e(f"s_cbranch_scc0 {L('masked')}")
     store_full(e, pairs)
@@ -432,35 +440,35 @@ def kernel_asm(pairs):
     return e.lines
 
 
-def emit_function(name, pairs):
-    lines = kernel_asm(pairs)
+def emit_function(name, pairs, totals=False):
+    lines = kernel_asm(pairs, totals)
     body = "\n".join(f'      "{ln}\\n"' for ln in lines)
-    clob_v = [f'"v{i}"' for i in range(0, V_ADMA)] + [f'"v{V_TMP}"']
+    clob_v = [f'"v{i}"' for i in range(64 if totals else 0, V_ADMA)] + [f'"v{V_TMP}"']
     clob_s = [f'"s{i}"' for i in range(60, 96)]
-    ins = ["[g0] \"s\"(g0)", "[g1] \"s\"(g1)", "[iters] \"s\"(iters)", "[phase] \"s\"(phase)", "[full] \"s\"(full)",
-           "[asoff] \"s\"(asoff)", "[bg] \"s\"(bg)", "[bc0] \"s\"(bc0)", "[bc1] \"s\"(bc1)", "[mg] \"s\"(mg)",
-           "[nbsb] \"s\"(nbsb)", "[nbsm] \"s\"(nbsm)", "[wavea] \"s\"(wavea)", "[waveb] \"s\"(waveb)",
-           "[wavem] \"s\"(wavem)", "[n8] \"s\"(n8)", "[M] \"s\"(M)", "[N] \"s\"(N)",
-           "[rA] \"s\"(rA)", "[rB] \"s\"(rB)", "[rM] \"s\"(rM)", "[rT] \"s\"(rT)"]
-    if pairs:
-        ins += ["[rCt] \"s\"(rCt)", "[ctoff] \"v\"(ctoff)"]
-    params = ("int g0, int g1, int iters, int phase, int full, int asoff, int bg, int bc0, int bc1, int mg, int nbsb, "
-              "int nbsm, int wavea, int waveb, int wavem, int n8, int M, int N, __amdgpu_buffer_rsrc_t rA, "
-              "__amdgpu_buffer_rsrc_t rB, __amdgpu_buffer_rsrc_t rM, __amdgpu_buffer_rsrc_t rT, int vadma0, "
-              "int vadma1, int vadma2, int vadma3, int vbdma, int vmdma, int vard0, int vard1, int vard2, int vard3, "
-              "int vbrd, int vmrd, int vst, int vrow, int vcol")
-    if pairs:
-        params += ", __amdgpu_buffer_rsrc_t rCt, int ctoff"
+    scalars = ["g0", "g1", "iters", "phase", "asoff", "bg", "bc0", "bc1", "mg", "nbsb", "nbsm", "wavea", "waveb", "wavem"]
+    scalars += ["ctup"] if totals else ["full", "n8", "M", "N"]
+    rsrc = ["rA", "rB", "rM"] + ([] if totals else ["rT"]) + (["rCt"] if pairs else [])
     pinned = [("vadma0", V_ADMA), ("vadma1", V_ADMA + 1), ("vadma2", V_ADMA + 2), ("vadma3", V_ADMA + 3),
               ("vbdma", V_BDMA), ("vmdma", V_MDMA), ("vard0", V_ARD), ("vard1", V_ARD + 1), ("vard2", V_ARD + 2),
-              ("vard3", V_ARD + 3), ("vbrd", V_BRD), ("vmrd", V_MRD), ("vst", V_ST), ("vrow", V_ROW), ("vcol", V_COL)]
-    outs = ", ".join(f'"+{{v{r}}}"({n})' for n, r in pinned)
+              ("vard3", V_ARD + 3), ("vbrd", V_BRD), ("vmrd", V_MRD)]
+    if not totals:
+        pinned += [("vst", V_ST), ("vrow", V_ROW), ("vcol", V_COL)]
+    ins = [f'[{n}] "s"({n})' for n in scalars + rsrc] + (['[ctoff] "v"(ctoff)'] if pairs else [])
+    params = [f"int {n}" for n in scalars] + [f"__amdgpu_buffer_rsrc_t {n}" for n in rsrc] + [f"int {n}" for n, _ in pinned]
+    params += ["int ctoff"] if pairs else []
+    outs = [f'"+{{v{r}}}"({n})' for n, r in pinned]
+    if totals:   # the lane's totals T(rs, jp, cs), two dwords each
+        params += ["v32i& t0", "v32i& t1"]
+        outs = ['"=&{v[0:31]}"(t0)', '"=&{v[32:63]}"(t1)'] + outs
+    what = "A16 as digit-row pairs (rows 2r = x >> 8, 2r + 1 = (x & 255) - 128; 256 hi + lo per group)" if pairs else "A8"
+    if totals:
+        what += "; the totals stay in registers"
     return f"""
-// {name}: {'A16 as digit-row pairs (rows 2r = x >> 8, 2r + 1 = (x & 255) - 128; 256 hi + lo per group)' if pairs else 'A8'}
-__device__ __forceinline__ void {name}({params}) {{
+// {name}: {what}
+__device__ __forceinline__ void {name}({", ".join(params)}) {{
   asm volatile(
 {body}
-      : {outs}
+      : {", ".join(outs)}
       : {", ".join(ins)}
       : {", ".join(clob_v)}, {", ".join(clob_s)}, "vcc", "scc", "memory");
 }}
@@ -473,9 +481,11 @@ def main():
            f"#define GEMM_ASM_LDS_BYTES {LDS_BYTES}",
            f"#define GEMM_ASM_B_BASE {B_BASE}",
            f"#define GEMM_ASM_M_BASE {M_BASE}",
-           f"#define GEMM_ASM_A_HI {A_STAGE[2]}"]
+           f"#define GEMM_ASM_A_HI {A_STAGE[2]}",
+           "typedef int v32i __attribute__((ext_vector_type(32)));"]
     out.append(emit_function("gemm_asm_main_a8", False))
     out.append(emit_function("gemm_asm_main_pairs", True))
+    out.append(emit_function("gemm_asm_main_pairs_totals", True, True))
     sys.stdout.write("\n".join(out) + "\n")
 
 

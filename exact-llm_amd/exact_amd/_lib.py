@@ -55,6 +55,8 @@ SIGNATURES = {
     "exact_logits_argmax_noalloc": [P, P, P, P, I32, I32, I32, P],
     "exact_advance": [P, I32, P],
     "exact_zero": [P, I64, P],
+    "exact_gemm_g128_digits_swiglu": [P, P, P, P, P, P, P, P, I32, I32, I32, P],
+    "exact_quant_slices": [P, P, I32, P, P, I32, I32, P, P],
     "exact_sample": [P, I32, I32, U64, P, I64, P, P, P, P],
     "exact_sample_split": [P, I32, I32, U64, P, I64, P, P, P, P, I64, P],
     "exact_router_topk": [P, I32, P, P, P, P, I32, P, P, I32, I32, I32, I32, P],
@@ -71,6 +73,7 @@ SIGNATURES = {
 }
 OTHER = {"exact_version": ([], ctypes.c_int), "exact_last_error": ([], ctypes.c_char_p),
          "exact_attention_decode_workspace": ([I32, I32, I32, I32, I32], ctypes.c_int64),
+         "exact_gemm_swiglu_supported": ([I32, I32, I32], ctypes.c_int),
          "exact_gemm_g128_splits": ([I32, I32, I32, I32], ctypes.c_int),
          "exact_sample_workspace": ([I32, I32], ctypes.c_int64),
          "exact_attention_prefill_workspace": ([I32, I32, I32, I32, I32], ctypes.c_int64)}

@@ -401,6 +401,9 @@ class TModel:
         # one per CU)
         fsfuse = (self.FFN_NORM and sfuse and qfuse and D > ops.NORM_SWIGLU_KMAX and D <= ops.NORM_SWIGLU_WIDE_KMAX
                   and c.I % 128 == 0)
+        # prompts whose gate|up GEMM splits no K: the SwiGLU in its epilogue (no totals in memory, no SwiGLU launch)
+        gsfuse = (group and not keep and not c.moe and self.abits == 15 and R > ops.A16_DIGIT_ROWS
+                  and ops.gemm_swiglu_supported(R, self.w.layers[0]["gateup"]))
         if ws.h is None and not c.moe and ((xfuse and (c.I > 8192 or nfuse or sfuse)) or sqfuse):
             ws.h = torch.zeros((R, ws.I), dtype=I64, device=self.dev)
         x_cur, x_nxt = ws.x, ws.x2
@@ -506,6 +509,10 @@ class TModel:
             elif sqfuse:
                 ops.gemv_swiglu(ws.xq, L["gateup"], ws.s, tab.silu, ws.h, ws.part_sw, t=t_gu if keep else None)
                 ops.quant_rows(ws.h, ws.part_sw, c.I // ops.SWIGLU_PART_COLS, self.abits, ws.hq, ws.sh, x8=dh)
+                self._lin(ws.hq, L["down"], t_d, x8=dh)
+                res_t, res_s = t_d, ws.sh
+            elif gsfuse:   # h takes the place of the totals, which this workspace then never holds
+                ops.gemm_swiglu_qrow(dx, L["gateup"], ws.s, tab.silu, t_gu, ws.part_sw, ws.hq, ws.sh, dh)
                 self._lin(ws.hq, L["down"], t_d, x8=dh)
                 res_t, res_s = t_d, ws.sh
             elif group:
@@ -627,8 +634,12 @@ class TModel:
             ops.gemv_qrow_acc(ws.hsh, ws.part_sw, c.SI // ops.SWIGLU_PART_COLS, self.abits, L["sd"], ws.t_sd, ws.ssh,
                               zero=zero)
         else:
-            self._lin(ws.xq, L["sgu"], ws.t_sgu, x8=dx)
-            ops.swiglu_qrow(ws.t_sgu, ws.s, tab.silu, self.abits, ws.shq, ws.ssh, clear=adds["sgu"], part=ws.part_sw, x8=dh)
+            if self.abits == 15 and ws.R > ops.A16_DIGIT_ROWS and ops.gemm_swiglu_supported(ws.R, L["sgu"]):
+                ops.gemm_swiglu_qrow(dx, L["sgu"], ws.s, tab.silu, ws.t_sgu, ws.part_sw, ws.shq, ws.ssh, dh)
+            else:
+                self._lin(ws.xq, L["sgu"], ws.t_sgu, x8=dx)
+                ops.swiglu_qrow(ws.t_sgu, ws.s, tab.silu, self.abits, ws.shq, ws.ssh, clear=adds["sgu"], part=ws.part_sw,
+                                x8=dh)
             self._lin(ws.shq, L["sd"], ws.t_sd, x8=dh)
             if zero is not None:
                 ops.zero_(zero)

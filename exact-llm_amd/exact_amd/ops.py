@@ -407,6 +407,25 @@ def swiglu_qrow(t, s, silu, bits=15, xq=None, sq=None, clear=False, part=None, h
     return xq, sq
 
 
+def gemm_swiglu_supported(R, lin):
+    """Whether gemm_swiglu_qrow takes R int16 rows of this gate|up linear."""
+    return (lin.mh is None and lin.bias is None and lin.N % 2 == 0
+            and _lib.load().exact_gemm_swiglu_supported(R, lin.N // 2, lin.K) == 1)
+
+
+def gemm_swiglu_qrow(x8, lin, s, silu, h, part, xq, sq, xq8=None):
+    """gemm_g128 of a gate|up linear on the digit rows x8 with the SwiGLU in its epilogue, then the qrow of its rows into
+    xq (int16), sq and the digit rows xq8: the results of swiglu_qrow on the linear's totals. h: (R, I) int64 and part:
+    (R, I / 32) int32 scratch."""
+    R, I = s.numel(), lin.N // 2
+    _need_packed(lin, "gemm_swiglu_qrow")
+    _lib.call("exact_gemm_g128_digits_swiglu", _digits(x8, R, lin.K), _ptr(lin.wp), _ptr(lin.mp), _ptr(colterm(lin)),
+              _ptr(_need(s, I32, "s", R)), _ptr(silu), _ptr(_need(h, I64, "h", R * I)),
+              _ptr(_need(part, I32, "part", R * (I // 32))), R, I, lin.K, _stream())
+    _lib.call("exact_quant_slices", _ptr(h), _ptr(part), 15, _ptr(_need(xq, I16, "xq", R * I)), _ptr(_need(sq, I32, "sq", R)), R,
+              I, _digits(xq8, R, I), _stream())
+
+
 def quant_rows(src, part, nparts, bits, xq, s, K=None, clear=False, x8=None, zero=None):
     """qrow of src rows (first K columns) given per-slice bit lengths of max |src| part (R, nparts) int32.
     x8: (2R, K) int8, also receives xq's digit rows. zero: an int64 tensor the launch also clears."""

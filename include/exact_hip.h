@@ -122,6 +122,19 @@ int exact_gemm_g128_zeroed(const void* x, int32_t abits, const int8_t* wp, const
  * that these entries refuse or run on another path, which may add. */
 int exact_gemm_g128_splits(int32_t abits, int32_t R, int32_t N, int32_t K);
 
+/* exact_gemm_g128_digits of a gate|up linear (2 I packed columns, gate first; no wide scales) with the SwiGLU in its epilogue:
+ * h = rs(isilu(rs(g, 28 - s[r])) * rs(u, 28 - s[r]), 16) (exact_llm.py:118-123) for R int16 rows given as digit rows x8.
+ * part (R, I / 32) receives the bit length of max |h| of each row's 32-column slice, and h (R, I, int64 slots, 16-byte
+ * aligned) its values: as int64, or, where part is at most 31, as int32 in the first half of the slice's slots.
+ * exact_quant_slices reads that form: xq (int16) and s as qrow (exact_llm.py:41-46), and the digit rows x8 unless NULL;
+ * bits 8..15, K % 32 == 0. exact_gemm_swiglu_supported: 1 for sizes the GEMM takes (others: EXACT_E_UNSUPPORTED). */
+int exact_gemm_swiglu_supported(int32_t R, int32_t I, int32_t K);
+int exact_gemm_g128_digits_swiglu(const int8_t* x8, const int8_t* wp, const int16_t* mp, const int64_t* colterm,
+                                  const int32_t* s, const int32_t* silu_t, int64_t* h, int32_t* part, int32_t R, int32_t I,
+                                  int32_t K, void* stream);
+int exact_quant_slices(const int64_t* h, const int32_t* part, int32_t bits, int16_t* xq, int32_t* s, int32_t R, int32_t K,
+                       int8_t* x8, void* stream);
+
 /* qrow fused into the GEMV that consumes it: t += qrow(xs, abits) . W (t holds zeros or a running total), where
  * row r of xs (int64, ldx apart) is quantised with s = max(max_i part[r * nparts + i] - abits, 0) and
  * part holds the producer's bit lengths of max |xs| over slices of the row (exact_attention's per-head

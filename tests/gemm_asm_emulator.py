@@ -386,13 +386,14 @@ def pack(W, M16, N, K):
     return Wp, Mp
 
 
-def inputs_for(bm, bn, wave, Mrows, N, K, pairs):
+def inputs_for(bm, bn, wave, Mrows, N, K, pairs, swiglu=False):
     """transcription of k_gemm_asm's set-up (gemm.hip)"""
     lane = np.arange(64)
     Gn, nbs = K // 128, (N + 63) // 64
     wm, wn = wave >> 1, wave & 1
     j, q = lane & 15, lane >> 4
-    row0, nb0 = bm * 256, bn * 2
+    row0, nb0 = bm * 256, bn if swiglu else bn * 2
+    up = nbs // 2
     col0 = nb0 * 64
     g0, g1 = 0, Gn
     iters = (g1 - g0 + 5) // 6
@@ -404,13 +405,17 @@ def inputs_for(bm, bn, wave, Mrows, N, K, pairs):
         gr = np.where(row0 + r < Mrows, row0 + r, Mrows - 1)
         vad.append(gr * K + c * 16)
     vbdma = (4 * (lane & 15) + (lane >> 4)) * 16
+    if swiglu:
+        vbdma = (32 * (wave >> 2) + 2 * (lane & 15) + (lane >> 4 & 1)) * 16 + (lane >> 5) * up * 8192
     bc = []
     for i in range(2):
         seg = wave * 2 + i
-        tl = (seg >> 3) if nb0 + (seg >> 3) < nbs else nbs - 1 - nb0
+        tl = 0 if swiglu else (seg >> 3) if nb0 + (seg >> 3) < nbs else nbs - 1 - nb0
         bc.append((nb0 + tl) * 8192 + (seg & 7) * 1024)
     ncol = (nbs - nb0) * 64
     vmdma = np.where(2 * lane < ncol, 2 * lane, ncol - 2) * 2
+    if swiglu:
+        vmdma = (32 * (lane >> 5) + (lane & 30)) * 2 + (lane & 1) * up * 128
     vard = [None] * 4
     for kh in range(2):
         vard[kh] = wm * 8192 + j * 128 + (((kh * 4 + q) ^ ((j >> 1) & 7)) << 4)
@@ -432,12 +437,17 @@ def inputs_for(bm, bn, wave, Mrows, N, K, pairs):
             "vrow": (G.V_ROW, orow), "vcol": (G.V_COL, ocol)}
     rsrc = {"rA": "A", "rB": "B", "rM": "M", "rT": "T", "rCt": "Ct"}
     inp = {"s": s, "vpin": vpin, "rsrc": rsrc}
+    if swiglu:
+        s["ctup"] = N * 4
+        ocol = col0 + 32 * wn + 2 * j
+        for n in ("vst", "vrow", "vcol"):
+            del vpin[n]
     if pairs:   # the asm's one compiler-placed VGPR input; emulated in a register the asm does not use
         inp["vpin"]["ctoff"] = (CTOFF_REG, np.where(ocol < N, ocol, 0) * 8)
     return inp
 
 
-def emulate(pairs, K, Mrows, N, seed=1, lines=None):
+def emulate(pairs, K, Mrows, N, seed=1, lines=None, swiglu=False):
     """(totals from the emulated kernel, int64 reference) for a seeded GEMM: int8 rows (A8) or the digit rows of
     int16 rows (pairs), clipped N(0, 40^2) int8 weights, positive int16 group scales"""
     rng = np.random.default_rng(seed)
@@ -458,11 +468,24 @@ def emulate(pairs, K, Mrows, N, seed=1, lines=None):
     mem = {"A": A8.reshape(-1).view(np.uint8).copy(), "B": Wp.view(np.uint8).copy(), "M": Mp.view(np.uint8).copy(),
            "T": Tmem, "Ct": ct.view(np.uint8).copy()}
     if lines is None:
-        lines = G.kernel_asm(pairs)
+        lines = G.kernel_asm(pairs, swiglu)
     lines = [ln.replace("%[ctoff]", f"v{CTOFF_REG}") for ln in lines]
     for bm in range((Mrows + 255) // 256):
         for bn in range((nbs + 1) // 2):
-            Block(lines, mem, [inputs_for(bm, bn, w, Mrows, N, K, pairs) for w in range(8)], Mrows, pairs).run()
+            blk = Block(lines, mem, [inputs_for(bm, bn, w, Mrows, N, K, pairs, swiglu) for w in range(8)], Mrows, pairs)
+            blk.run()
+            if swiglu:   # the totals left in v0..v63, where swiglu_epilogue takes them from
+                Tv = Tmem[:Mout * N * 8].view(np.int64).reshape(Mout, N)
+                for w in blk.waves:
+                    for lane in range(64):
+                        wm, wn, j, q = w.id >> 1, w.id & 1, lane & 15, lane >> 4
+                        for k in range(8):
+                            row = bm * 128 + wm * 32 + 2 * q + 8 * (k >> 1) + (k & 1)
+                            for cs in range(4):
+                                col = bn * 64 + 32 * wn + 2 * j + (cs & 1) + (cs >> 1) * (N // 2)
+                                r = 2 * (4 * k + cs)
+                                if row < Mout:
+                                    Tv[row, col] = np.int64(w.v[r, lane]) | (np.int64(w.v[r + 1, lane].view(np.int32)) << 32)
     T = Tmem[:Mout * N * 8].view(np.int64).reshape(Mout, N)
     ref = np.zeros((Mout, N), np.int64)
     for g in range(Gn):

@@ -23,6 +23,13 @@ def test_generated_gemm_matches_int64_matmul(pairs, K, Mrows, N):
     assert np.array_equal(T, ref)
 
 
+@pytest.mark.parametrize("K,Mrows,N", [(128, 256, 128), (768, 300, 256), (1664, 140, 384)])
+def test_totals_variant_leaves_gate_and_up_columns_in_one_lane(K, Mrows, N):
+    """the main loop of the SwiGLU GEMM: gate tile and up tile halves side by side, totals left in registers"""
+    T, ref = E.emulate(True, K, Mrows, N, seed=K + Mrows + N, swiglu=True)
+    assert np.array_equal(T, ref)
+
+
 def test_emulator_fails_a_dropped_lds_wait(monkeypatch):
     monkeypatch.setattr(G.Emit, "need", lambda self, regs: None)
     with pytest.raises(E.Race):

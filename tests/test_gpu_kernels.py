@@ -629,3 +629,35 @@ def test_gemv_large_a8_partial_row_block(thr, R, N, K):
     acc = dev(t0, I64)
     ops.gemv_g128_acc(dev(xq, I8), 7, lin, acc)
     assert np.array_equal(host(acc), exp + t0)
+
+
+@pytest.mark.parametrize("R,I,K", [(65, 64, 128), (128, 1024, 256), (129, 704, 256), (300, 448, 384), (515, 1088, 896)])
+def test_swiglu_in_the_prefill_gemm_matches_its_separate_launches(thr, R, I, K):
+    """Ragged and whole row tiles; row shifts from 0 to past 28, so that slices of h are held in 32 and in 64 bits, gates
+    lie inside and outside the table, and the totals are shifted right and left"""
+    lin, kw, km = synth_lin(thr, 91, "gu", 2 * I, K)
+    assert ops.gemm_swiglu_supported(R, lin)
+    r = np.random.default_rng(R + I)
+    xq = r.integers(-32767, 32768, (R, K)) >> r.integers(0, 14, (R, 1))
+    x8 = dev(np.stack([xq >> 8, (xq & 255) - 128], 1).reshape(2 * R, K), I8)
+    sh = r.integers(0, 26, R)
+    sh[::17] = 30
+    s = dev(sh, I32)
+    from exact_amd.tables import DeviceTables
+    tab = DeviceTables(DEV, 1, 64, 1e6)
+    z = lambda *n, dt: torch.full(n, 99, dtype=dt, device=DEV)
+    h, part = z(R, I, dt=I64), z(R, I // 32, dt=I32)
+    xa, sa, da = z(R, I, dt=I16), z(R, dt=I32), z(2 * R, I, dt=I8)
+    ops.gemm_swiglu_qrow(x8, lin, s, tab.silu, h, part, xa, sa, da)
+    t = ops.gemm_g128(dev(xq, I16), 15, lin)
+    xb, sb, db = z(R, I, dt=I16), z(R, dt=I32), z(2 * R, I, dt=I8)
+    hb = z(R, I, dt=I64)
+    ops.swiglu_qrow(t, s, tab.silu, 15, xb, sb, part=ops.swiglu_parts(R, I, DEV), h=hb, x8=db)
+    assert torch.equal(sa, sb) and torch.equal(xa, xb) and torch.equal(da, db)
+    ot = oracle_t(xq[:40], synth.weights_np(kw, 2 * I, K), synth.scales_np(km, 2 * I, K))
+    y = [O.round_shift(ot[i], int(28 - sh[i])) for i in range(40)]
+    for i in range(40):   # and against the oracle
+        q, e = O.qrow(O.round_shift(O.isilu(y[i][:I]) * y[i][I:], 16)[None], 15)
+        assert np.array_equal(host(xa)[i], q[0]) and int(host(sa)[i]) == int(np.ravel(e)[0]), i
+    pn = host(part)
+    assert (pn <= 31).any() and (pn > 31).any()
