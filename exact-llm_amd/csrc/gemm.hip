@@ -312,10 +312,11 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void k_gemm_a8p(const int8_t* __re
                                                      int tiles_m, int tiles_n, int ksplit, int use_atomic,
                                                      const int64_t* __restrict__ colterm, const int32_t* __restrict__ chunk_e,
                                                      const int32_t* __restrict__ chunk_p0, const int32_t* __restrict__ chunk_n,
-                                                     const int32_t* __restrict__ nchunks, int64_t w_stride, int64_t m_stride) {
+                                                     const int32_t* __restrict__ nchunks, int64_t w_stride, int64_t m_stride,
+                                                     const int32_t* __restrict__ row_map) {
   using C = GemmCfg<7, WM, WN, S>;
   static_assert(EXACT_TILE_GN, "the block's tiles of one group are contiguous in the group-major layout");
-  static_assert(C::BN == 128, "one dword copy per lane covers the block's 128 scales");
+  static_assert(C::BN <= 128, "one dword copy per lane covers the block's scales");
   constexpr int SMW = WIDE ? 512 : 256;                     // each wave keeps its own copy of the scales
   constexpr int SM_BYTES = C::WAVES * SMW;
   constexpr int STAGE = C::A_BYTES + C::B_BYTES + SM_BYTES;
@@ -362,7 +363,8 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void k_gemm_a8p(const int8_t* __re
   for (int i = 0; i < C::A_KB_PER_WAVE; ++i) {
     const int seg = wave * C::A_KB_PER_WAVE + i;            // 1 KiB LDS segment = 8 rows x 128 bytes
     const int r = seg * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-    const int gr = row0 + r < Mlim ? row0 + r : Mlim - 1;   // rows past the tile's rows read a valid row, never stored
+    int gr = row0 + r < Mlim ? row0 + r : Mlim - 1;   // rows past the tile's rows read a valid row, never stored
+    if (GROUPED && row_map) gr = PAIRS ? 2 * row_map[gr >> 1] + (gr & 1) : row_map[gr];   // the pair's activation row
     aoffs[i] = (uint32_t)gr * (uint32_t)K + (uint32_t)(c * 16);
   }
   const int moff = (2 * lane < ncol ? 2 * lane : ncol - 2) * 2;
@@ -725,27 +727,26 @@ __global__ __launch_bounds__(256) void k_split_rows_a16(const int16_t* __restric
 }
 
 // gathered int8 rows: x8[p] = x[row_map[p]] (16 bytes per thread; K % 16 == 0)
-__global__ __launch_bounds__(256) void k_gather_rows_a8(const int8_t* __restrict__ x, int8_t* __restrict__ x8, int64_t P, int K,
-                                                        const int32_t* __restrict__ row_map) {
-  const int64_t n16 = P * (K / 16);
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n16; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t p = i / (K / 16), c = (i - p * (K / 16)) * 16;
-    *reinterpret_cast<v4i*>(x8 + p * K + c) = *reinterpret_cast<const v4i*>(x + (int64_t)row_map[p] * K + c);
-  }
-}
+// Tile of the A8 kernel by its A rows M (digit rows of int16): up to 64 rows (prompts of 17 to 32 tokens) 64 x 64, one wave, three
+// blocks a CU; up to 128 rows 128 x 128, two blocks a CU; 256 x 128 beyond. 37888 x 3584 at 32 tokens: 31.4 us in 64 x 64, 40.0
+// in 64 x 128, 40.3 in 128 x 128, whose waves of padding rows compute as well; at 41 tokens 60.0, 56.6 and 40.3.
+static int gemm_tile_rows(int64_t M) { return M <= 64 ? 64 : M <= GEMM_SMALL_M ? 128 : 256; }
+static int64_t gemm_tiles(int64_t M, int64_t N) { return cdiv(M, gemm_tile_rows(M)) * cdiv(cdiv(N, 64), M <= 64 ? 1 : 2); }
 
 // K splits of a GEMM on the A8 kernel: blocks that walk fewer groups each, against every split adding its own R x N 64-bit
-// totals. us by group walked and by 10^6 atomic adds, from sweeps over 14 shapes of N 896..37888 and K 896..18944 at 17 to
-// 253 output rows: 0.8 in 128-row tiles, 0.52 in 256-row tiles, and 4.7. Never more blocks than CUs (a split just past one
-// block a CU is slower than the one before: 40 column tiles at 41 rows 15.3 us in 6 splits, 17.8 in 7). Powers of two that
-// kept 8 groups a block, used before: 4608 x 3584 at 41 rows 16.9 us (2 splits), now 12.5 (5); 2048 x 2048 at 41 rows 10.6
-// and 7.4; 6144 x 2048 at 253 rows 27.6 (2) and 20.9 (none: the split cost more than it gave).
-static int gemm_ksplit(int tiles, int G, int64_t rows, int64_t N, bool tiles128, bool zeroed) {
-  const double group = tiles128 ? 0.8 : 0.52, add = 4.7e-6 * (double)rows * (double)N;
-  const double clear = zeroed ? 0.0 : 1.2 + (double)rows * (double)N * 8 / 4e6;   // t's zero fill: one more launch
+// totals. us by group walked and by 10^6 atomic adds, fitted to sweeps over 19 shapes of N 61..37888 and K 896..18944 at 17 to
+// 1000 output rows (the choice is within 1.1% of the fastest split on average): 0.7 in 128-row tiles, else 0.6, and 4.7. Never
+// more blocks than CUs (a split just past one block a CU is slower than the one before: 40 column tiles at 41 rows 15.3 us in 6
+// splits, 17.8 in 7), in 64-row tiles than three a CU. Powers of two that kept 8 groups a block, used before: 4608 x 3584 at 41
+// rows 16.9 us (2 splits), now 12.5 (5); 2048 x 2048 at 41 rows 10.6 and 7.4; 6144 x 2048 at 253 rows 27.6 (2) and 20.9 (none:
+// the split cost more than it gave).
+static int gemm_ksplit(int64_t M, int64_t rows, int64_t N, int G, bool zeroed) {
+  const int64_t tiles = gemm_tiles(M, N), most = M <= 64 ? 768 : 256;
+  const double group = gemm_tile_rows(M) == 128 ? 0.7 : 0.6, add = 4.7e-6 * (double)rows * (double)N;
+  const double clear = zeroed ? 0.0 : 0.6 + (double)rows * (double)N * 8 / 4e6;   // t's zero fill: one more launch
   int best = 1;
   double cost = group * G + add;
-  for (int k = 2; k <= G && (int64_t)tiles * k <= 256; ++k) {
+  for (int k = 2; k <= G && tiles * k <= most; ++k) {
     const double c = group * ((G + k - 1) / k) + add * k + clear;
     if (c < cost) {
       cost = c;
@@ -831,7 +832,7 @@ static bool gemm_swiglu_ok(int64_t R, int64_t I, int64_t K) {
   if (R <= 0 || I <= 0 || K <= 0 || K % 128 || I % 64 || 2 * R <= GEMM_SMALL_M || 2 * R * K >= (1LL << 32)) return false;
   const int64_t G = K / 128, nbs = 2 * I / 64, tiles = cdiv(2 * R, 256) * (I / 64);
   if (!GEMM_ASM || GEMM_KSPLIT > 1 || G * nbs * 8192 >= (1LL << 32) || tiles > INT32_MAX / 2) return false;
-  return tiles > 256 || gemm_ksplit((int)tiles, (int)G, R, 2 * I, false, true) == 1;
+  return gemm_ksplit(2 * R, R, 2 * I, (int)G, true) == 1;
 }
 
 // M: rows of the A operand (digit rows when PAIRS: the output has M / 2 rows, written through colterm)
@@ -850,7 +851,7 @@ static int gemm_launch_a8p_t(const void* x, const int8_t* wp, const int16_t* mp,
   const int G = K / 128, nbs = (N + 63) / 64;
   const int tiles_m = (M + C::BM - 1) / C::BM, tiles_n = (nbs + C::NT - 1) / C::NT;
   int ksplit = ksplit_req;
-  if (ksplit <= 0) ksplit = gemm_ksplit(tiles_m * tiles_n, G, PAIRS ? M / 2 : M, N, WM == 2, zeroed);
+  if (ksplit <= 0) ksplit = gemm_ksplit(M, PAIRS ? M / 2 : M, N, G, zeroed);
   if (ksplit > G) ksplit = G;
   // (exact_gemm_g128_splits repeats this choice)
   // one K pass over enough tiles: the assembly main loop (same tiles and outputs; 32-bit offsets into x, W and t)
@@ -866,13 +867,13 @@ static int gemm_launch_a8p_t(const void* x, const int8_t* wp, const int16_t* mp,
   const int grid = ((nblk + 7) / 8) * 8;
   hipLaunchKernelGGL((k_gemm_a8p<WM, WN, S, PAIRS, WIDE>), dim3(grid), dim3(C::THREADS), lds, st,
                      reinterpret_cast<const int8_t*>(x), wp, mp, mh, t, M, N, K, G, nbs, tiles_m, tiles_n, ksplit, use_atomic,
-                     colterm, nullptr, nullptr, nullptr, nullptr, (int64_t)0, (int64_t)0);
+                     colterm, nullptr, nullptr, nullptr, nullptr, (int64_t)0, (int64_t)0, nullptr);
   return launch_status("gemm_g128");
 }
 
 // MoE experts: one grouped launch over the dispatched chunks (row tile = chunk), max_chunks row tiles
 template <int WM, int WN, int S, bool PAIRS>
-static int gemm_launch_experts(const int8_t* x8, const int8_t* wp, const int16_t* mp, int64_t w_stride, int64_t m_stride,
+static int gemm_launch_experts(const int8_t* x8, const int32_t* row_map, const int8_t* wp, const int16_t* mp, int64_t w_stride, int64_t m_stride,
                                const int64_t* colterm, const int32_t* chunk_e, const int32_t* chunk_p0,
                                const int32_t* chunk_n, const int32_t* nchunks, int max_chunks, int64_t* t, int M, int N,
                                int K, hipStream_t st) {
@@ -890,16 +891,19 @@ static int gemm_launch_experts(const int8_t* x8, const int8_t* wp, const int16_t
   const int grid = ((nblk + 7) / 8) * 8;
   hipLaunchKernelGGL((k_gemm_a8p<WM, WN, S, PAIRS, false, true>), dim3(grid), dim3(C::THREADS), lds, st, x8, wp, mp, nullptr, t,
                      M, N, K, G, nbs, max_chunks, tiles_n, 1, 0, colterm, chunk_e, chunk_p0, chunk_n, nchunks, w_stride,
-                     m_stride);
+                     m_stride, row_map);
   return launch_status("gemm_g128_experts");
 }
 
 template <int WM, int WN, int S, bool PAIRS = false>
 static int gemm_launch_a8p(const void* x, const int8_t* wp, const int16_t* mp, const int16_t* mh, int64_t* t, int M, int N,
                            int K, hipStream_t st, int ksplit_req, const int64_t* colterm = nullptr, bool zeroed = false) {
-  // up to 128 rows (prompts of 49-64 tokens as int16 digit rows): 128-row tiles, two 4-wave blocks per CU, instead
-  // of 256-row tiles half of padding
-  if (M <= GEMM_SMALL_M && WM != 2) {
+  const int rows = gemm_tile_rows(M);
+  if (rows == 64) {
+    if (mh) return gemm_launch_a8p_t<1, 1, 3, PAIRS, true>(x, wp, mp, mh, t, M, N, K, st, ksplit_req, colterm, zeroed);
+    return gemm_launch_a8p_t<1, 1, 3, PAIRS, false>(x, wp, mp, nullptr, t, M, N, K, st, ksplit_req, colterm, zeroed);
+  }
+  if (rows == 128) {
     if (mh) return gemm_launch_a8p_t<2, WN, 2, PAIRS, true>(x, wp, mp, mh, t, M, N, K, st, ksplit_req, colterm, zeroed);
     return gemm_launch_a8p_t<2, WN, 2, PAIRS, false>(x, wp, mp, nullptr, t, M, N, K, st, ksplit_req, colterm, zeroed);
   }
@@ -969,21 +973,28 @@ extern "C" int exact_gemm_g128_experts(const void* x, int32_t abits, const int32
   const int64_t rows = (abits == 15 ? 2 : 1) * (int64_t)P;
   if (rows * K >= (1LL << 32)) return EXACT_E_UNSUPPORTED;   // 32-bit buffer offsets
   hipStream_t st = as_stream(stream);
-  const int64_t n16 = (int64_t)P * (K / 16);
-  const int blocks = (int)std::min<int64_t>((n16 + 255) / 256, 8192);
   if (abits == 15) {
+    const int blocks = (int)std::min<int64_t>(((int64_t)P * (K / 16) + 255) / 256, 8192);
     hipLaunchKernelGGL(k_split_rows_a16, dim3(blocks), dim3(256), 0, st, static_cast<const int16_t*>(x), x8, (int64_t)P, K,
                        row_map);
-    return gemm_launch_experts<GEMM_A8P_CFG, true>(x8, wp, mp, w_stride, m_stride, colterm, chunk_e, chunk_p0, chunk_n,
+    return gemm_launch_experts<GEMM_A8P_CFG, true>(x8, nullptr, wp, mp, w_stride, m_stride, colterm, chunk_e, chunk_p0, chunk_n,
                                                    nchunks, max_chunks, t, (int)rows, N, K, st);
   }
-  const int8_t* xa = static_cast<const int8_t*>(x);
-  if (row_map) {
-    hipLaunchKernelGGL(k_gather_rows_a8, dim3(blocks), dim3(256), 0, st, xa, x8, (int64_t)P, K, row_map);
-    xa = x8;
-  }
-  return gemm_launch_experts<GEMM_A8P_CFG, false>(xa, wp, mp, w_stride, m_stride, nullptr, chunk_e, chunk_p0, chunk_n, nchunks,
-                                                  max_chunks, t, (int)rows, N, K, st);
+  return gemm_launch_experts<GEMM_A8P_CFG, false>(static_cast<const int8_t*>(x), row_map, wp, mp, w_stride, m_stride, nullptr,
+                                                  chunk_e, chunk_p0, chunk_n, nchunks, max_chunks, t, (int)rows, N, K, st);
+}
+
+extern "C" int exact_gemm_g128_experts_digits(const int8_t* x8, const int32_t* row_map, const int8_t* wp, const int16_t* mp,
+                                              int64_t w_stride, int64_t m_stride, const int64_t* colterm, const int32_t* chunk_e,
+                                              const int32_t* chunk_p0, const int32_t* chunk_n, const int32_t* nchunks,
+                                              int32_t max_chunks, int64_t* t, int32_t P, int32_t N, int32_t K, void* stream) {
+  if (!x8 || !wp || !mp || !colterm || !chunk_e || !chunk_p0 || !chunk_n || !nchunks || !t) return EXACT_E_ARG;
+  if (P <= 0 || N <= 0 || K <= 0 || max_chunks <= 0 || w_stride <= 0 || m_stride <= 0) return EXACT_E_ARG;
+  if (K % 128 || (reinterpret_cast<uintptr_t>(x8) & 15) || (reinterpret_cast<uintptr_t>(wp) & 15) || (w_stride & 15) ||
+      2 * (int64_t)P * K >= (1LL << 32))
+    return EXACT_E_UNSUPPORTED;
+  return gemm_launch_experts<GEMM_A8P_CFG, true>(x8, row_map, wp, mp, w_stride, m_stride, colterm, chunk_e, chunk_p0, chunk_n,
+                                                 nchunks, max_chunks, t, 2 * P, N, K, as_stream(stream));
 }
 
 static int gemm_a16_entry(const int16_t* x, const int8_t* wp, const int16_t* mp, const int16_t* mh,
@@ -1023,9 +1034,7 @@ extern "C" int exact_gemm_g128_splits(int32_t abits, int32_t R, int32_t N, int32
   const int64_t M = (abits == 15 ? 2 : 1) * (int64_t)R;
   if ((abits != 15 && abits != 7) || R <= 16 || N <= 0 || K <= 0 || K % 128 || M * K >= (1LL << 32)) return 0;
   if (GEMM_KSPLIT > 0) return GEMM_KSPLIT;
-  const int64_t tiles_m = cdiv(M, M <= GEMM_SMALL_M ? 128 : 256), tiles_n = cdiv(cdiv(N, 64), 2);
-  if (tiles_m * tiles_n > 256) return 1;
-  return gemm_ksplit((int)(tiles_m * tiles_n), K / 128, R, N, M <= GEMM_SMALL_M, true);
+  return gemm_ksplit(M, R, N, K / 128, true);
 }
 
 extern "C" int exact_gemm_swiglu_supported(int32_t R, int32_t I, int32_t K) { return gemm_swiglu_ok(R, I, K); }

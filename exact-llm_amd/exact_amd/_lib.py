@@ -64,6 +64,7 @@ SIGNATURES = {
     "exact_moe_route": [P, I32, P, P, P, P, I32, P, P, I32, I32, I32, I32, P, P, P, P, P, P, P, I32, P],
     "exact_gemv_g128_experts": [P, I32, P, P, P, I64, I64, P, P, P, P, I32, P, I32, I32, P],
     "exact_gemm_g128_experts": [P, I32, P, P, P, I64, I64, P, P, P, P, P, P, I32, P, I32, I32, I32, P],
+    "exact_gemm_g128_experts_digits": [P, P, P, P, I64, I64, P, P, P, P, P, I32, P, I32, I32, I32, P],
     "exact_gemv_g128_experts_swiglu": [P, P, P, P, I64, I64, P, P, P, P, I32, I32, P, P, P, P, I32, I32, P],
     "exact_gemv_g128_experts_qrow_acc": [P, I64, P, I32, P, P, I64, I64, P, P, P, P, I32, I32, P, P, I32, I32, P],
     "exact_moe_swiglu_pair": [P, P, P, P, I64, I64, P, P, P, P, I32, I32, P, P, P, P, I32, P, P, P, P, P, P, I32, I32, I32, P],

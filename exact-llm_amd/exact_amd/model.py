@@ -234,6 +234,8 @@ class Workspace:
         if abits == 15 and R > ops.A16_DIGIT_ROWS:
             hmax = max(I, cfg.SI if cfg.moe else 0)
             self.dig = dict(x=z(2 * R, D, dt=I8), a=z(2 * R, H * hd, dt=I8), h=z(2 * R, hmax, dt=I8))
+            if cfg.moe:
+                self.dig["eh"] = z(2 * R * cfg.topk, cfg.MI, dt=I8)   # of the routed experts' rows, by pair
         if cfg.moe:
             k, P = cfg.topk, R * cfg.topk
             # chunk arrays for the smallest chunks this workspace may be dispatched with (the fused decode GEMVs' 4 pairs)
@@ -618,14 +620,18 @@ class TModel:
             ops.gemv_experts_qrow_acc(ws.eh, ws.part_eh, c.MI // ops.SWIGLU_PART_COLS, L["edown"], ws.disp, ws.t_ed,
                                       ws.esh)
         elif grouped:
-            ops.gemm_experts(ws.xq, self.abits, ws.disp["pair_row"], L["egu"], ws.disp, ws.t_egu, P)
+            # int16 rows above 16: their digit rows (of the norm, and of the SwiGLU's qrow), read by pair
+            xd = ws.xq if dx is None else ops.DigitRows(dx)
+            ops.gemm_experts(xd, self.abits, ws.disp["pair_row"], L["egu"], ws.disp, ws.t_egu, P)
         else:
             ops.gemv_experts(ws.xq, self.abits, ws.disp["pair_row"], L["egu"], ws.disp, ws.t_egu)
         if not efuse:
+            edig = ws.dig["eh"] if grouped and ws.dig is not None else None
             ops.swiglu_qrow(ws.t_egu, ws.disp["s_pair"], tab.silu, self.abits, ws.ehq, ws.esh, clear=not grouped,
-                            part=ws.part_esw)
+                            part=ws.part_esw, x8=edig)
             if grouped:
-                ops.gemm_experts(ws.ehq, self.abits, None, L["edown"], ws.disp, ws.t_ed, P)
+                hd = ws.ehq if edig is None else ops.DigitRows(edig)
+                ops.gemm_experts(hd, self.abits, None, L["edown"], ws.disp, ws.t_ed, P)
             else:
                 ops.gemv_experts(ws.ehq, self.abits, None, L["edown"], ws.disp, ws.t_ed)
         if sfuse:

@@ -784,9 +784,26 @@ def expert_colterm(lin):
     return ct
 
 
+class DigitRows:
+    """Interleaved int8 digit rows (2 R, K) of R int16 rows, as their producer wrote them."""
+
+    def __init__(self, x8):
+        self.x8 = _need(x8, I8, "x8")
+        self.shape = (x8.shape[0] // 2, x8.shape[1])
+
+
 def gemm_experts(x, abits, row_map, lin, disp, out, P):
     """out[p] = x[row_map[p]] . W_{expert of p} for the P dispatched pairs on the matrix cores; disp must come from
-    moe_dispatch with chunk = EXPERT_CHUNK[abits] (row_map None: x row p)."""
+    moe_dispatch with chunk = EXPERT_CHUNK[abits] (row_map None: x row p). x: rows, or DigitRows of int16 rows (at most P)."""
+    if isinstance(x, DigitRows):
+        _need(out, I64, "out", P * lin.N)
+        if abits != 15 or x.shape[1] != lin.K or out.shape[1] != lin.N or x.shape[0] > P or (row_map is None and x.shape[0] < P):
+            raise ExactError(f"gemm_experts: digit rows of {x.shape}, out {tuple(out.shape)} against ({lin.N}, {lin.K}), {P} pairs")
+        _lib.call("exact_gemm_g128_experts_digits", _ptr(x.x8), _ptr(row_map), _ptr(lin.wp), _ptr(lin.mp), lin.w_stride,
+                  lin.m_stride, _ptr(expert_colterm(lin)), _ptr(disp["chunk_e"]), _ptr(disp["chunk_p0"]), _ptr(disp["chunk_n"]),
+                  _ptr(disp["nchunks"]), min(disp["chunk_e"].numel(), -(-P // EXPERT_CHUNK[abits]) + lin.NE), _ptr(out), P, lin.N,
+                  lin.K, _stream())
+        return out
     _need(x, I16 if abits == 15 else I8, "x")
     _need(out, I64, "out", P * lin.N)
     if x.shape[1] != lin.K or out.shape[1] != lin.N:

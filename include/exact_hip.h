@@ -176,12 +176,19 @@ int exact_gemv_g128_norm_swiglu(const int64_t* x_in, int64_t* x_out, const int64
  * dispatched pairs, t[p] = x[row_map[p]] . W_e with e = chunk_e[c] (row_map NULL: x row p), expert e's packed
  * linear at wp + e * w_stride, mp + e * m_stride. int16 x runs as interleaved digit rows (as
  * exact_gemm_g128_a16) and needs colterm (NE, N) = each expert's sum_g colsum_g M_g. x8: workspace of 2 P K
- * (int16) or P K (int8, with row_map) bytes. max_chunks: the length of the chunk arrays (launch size).
+ * (int16) or P K (int8; not used) bytes. max_chunks: the length of the chunk arrays (launch size).
  * Replaces the per-expert loop of MoEInt.moe (moe_exact_kaggle.py:460-464) for prefill-sized pair counts. */
 int exact_gemm_g128_experts(const void* x, int32_t abits, const int32_t* row_map, const int8_t* wp, const int16_t* mp,
                             int64_t w_stride, int64_t m_stride, const int64_t* colterm, int8_t* x8, const int32_t* chunk_e,
                             const int32_t* chunk_p0, const int32_t* chunk_n, const int32_t* nchunks, int32_t max_chunks,
                             int64_t* t, int32_t P, int32_t N, int32_t K, void* stream);
+
+/* exact_gemm_g128_experts of int16 rows given as their interleaved digit rows (x8: rows 2 r, 2 r + 1 of activation row r, at
+ * most P of them): the GEMM reads row row_map[p] itself (NULL: row p), with no launch that splits the rows. */
+int exact_gemm_g128_experts_digits(const int8_t* x8, const int32_t* row_map, const int8_t* wp, const int16_t* mp,
+                                   int64_t w_stride, int64_t m_stride, const int64_t* colterm, const int32_t* chunk_e,
+                                   const int32_t* chunk_p0, const int32_t* chunk_n, const int32_t* nchunks, int32_t max_chunks,
+                                   int64_t* t, int32_t P, int32_t N, int32_t K, void* stream);
 
 /* The int16 (A16) GEMM on the int8 matrix cores as interleaved digit rows: x is split into rows
  * x8[2r] = x[r] >> 8 and x8[2r + 1] = (x[r] & 255) - 128 (exact_torch.py:101-102), the A8 GEMM runs on the

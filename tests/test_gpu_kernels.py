@@ -73,7 +73,7 @@ def test_gemm_rows(thr, abits, R):
 
 
 @pytest.mark.parametrize("abits", [15, 7])
-@pytest.mark.parametrize("R,N,K", [(17, 61, 2048), (19, 130, 128), (33, 200, 896), (64, 1152, 896), (65, 1152, 1664),
+@pytest.mark.parametrize("R,N,K", [(17, 61, 2048), (19, 130, 128), (32, 1152, 1664), (33, 200, 896), (64, 1152, 896), (65, 1152, 1664),
                                    (129, 328, 4864), (253, 64, 1408), (300, 1000, 256)])
 def test_gemm_k_splits(thr, abits, R, N, K):
     """K splits of uneven length (1 to 38 of them, in both tile sizes), whole output, into a cleared and an uncleared t; where

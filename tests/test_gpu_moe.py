@@ -439,3 +439,19 @@ def test_moe_pairs_match_the_separate_launches(tab, R, NE, k, MI, SI, K, D):
     for a, b, name in zip(outs[0], outs[1], ("eh", "epart", "sh", "spart", "et", "es", "st", "ss", "zero")):
         assert np.array_equal(a, b), name
     assert not outs[1][8].any()
+
+
+@pytest.mark.parametrize("R,NE,k,N,K", [(17, 8, 4, 200, 256), (130, 4, 2, 64, 384)])
+def test_expert_gemm_of_digit_rows_matches_int16_rows(R, NE, k, N, K):
+    """digit rows read by pair (row_map), and in dispatched order, against the GEMM that splits the int16 rows itself"""
+    rng = np.random.default_rng(R)
+    lin, e_sel, _, _, x = _expert_case(rng, 15, R, NE, k, N, K, list(range(NE)))
+    P = R * k
+    xd = dev(x, torch.int16)
+    d = _dispatch(e_sel, NE, k, ops.EXPERT_CHUNK[15], 15)
+    want, got, ordered = (torch.full((P, N), f, dtype=I64, device=DEV) for f in (-1, -2, -3))
+    ops.gemm_experts(xd, 15, d["pair_row"], lin, d, want, P)
+    split = lambda a: ops.DigitRows(dev(np.stack([a >> 8, (a & 255) - 128], 1).reshape(2 * len(a), K), torch.int8))
+    ops.gemm_experts(split(x), 15, d["pair_row"], lin, d, got, P)
+    ops.gemm_experts(split(x[host(d["pair_row"])]), 15, None, lin, d, ordered, P)
+    assert torch.equal(want, got) and torch.equal(want, ordered)
