@@ -45,6 +45,7 @@ SIGNATURES = {
     "exact_isoftmax": [P, P, P, P, I32, I32, P],
     "exact_qkv_rope_cache": [P, P, P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, I32, I32, P],
     "exact_attention": [P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, I32, I32, P],
+    "exact_attention_rows": [P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, I32, I32, I32, P],
     "exact_attention_qkv": [P, P, P, P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, I32, I32, P],
     "exact_attention_qkv_split": [P, P, P, P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, I32, I32, I32, P],
     "exact_attention_decode": [P, P, P, P, P, P, P, P, P, P, P, P, P, I32, P, I64, I32, I32, I32, I32, I32, I32, P],

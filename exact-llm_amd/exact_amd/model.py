@@ -223,6 +223,7 @@ class Workspace:
         # next decode step consumes them with no copy launch in between
         self.next_ids = self.ids
         self.seq = None   # (slot, keys) when the rows are one sequence's consecutive positions (prefill)
+        self.nkeys = None   # ... and a bound on the rows' positions
         self.h = None     # (R, I) SwiGLU values when the gate|up totals must stay intact (trace capture)
         self.hsh = None   # (R, SI) SwiGLU values of the MoE shared expert (decode rows)
         self.att_work = None   # of decode attention split over the keys
@@ -454,7 +455,8 @@ class TModel:
                     ops.attention_prefill(ws.qq, ws.sq, cache, ws.seq[0], ws.pos, ws.seq[1], tab.exp, ws.att, H, KV, hd,
                                           tab.inv, self._prefill_ws(R), ws.obits)
                 else:
-                    ops.attention(ws.qq, ws.sq, cache, ws.slot, ws.pos, tab.exp, ws.att, H, KV, hd, tab.inv, ws.obits)
+                    ops.attention(ws.qq, ws.sq, cache, ws.slot, ws.pos, tab.exp, ws.att, H, KV, hd, tab.inv, ws.obits,
+                                  nkeys=ws.nkeys)
             if nfuse:   # also clears the down totals the q|k|v GEMV read as its residual (t_qkv and t_d are one range)
                 ops.gemv_qrow_acc(ws.att, ws.obits, nob, self.abits, L["o"], t_o, ws.sa, zero=ws.t_qd if clear else None)
             elif xfuse:   # clears the q|k|v totals attention left (and, q|k|v norm-fused, the down totals it read)
@@ -676,6 +678,7 @@ class TModel:
         ws.pos.copy_(torch.arange(p0, p0 + T, dtype=I32))
         # the matrix-core attention for prefill chunks of PREFILL_MIN_ROWS[hd] rows or more (hd 64, 128); the row kernel otherwise
         ws.seq = (slot, p0 + T) if T >= self.PREFILL_MIN_ROWS.get(self.cfg.hd, 1 << 30) else None
+        ws.nkeys = p0 + T
         key = (T, id(cache), slot, p0, bool(last_only))
         g = self._graphs.get(key) if graph else None
         try:
@@ -692,7 +695,7 @@ class TModel:
                     while len(self._graphs) > self.PREFILL_GRAPHS:
                         self._graphs.popitem(last=False)
         finally:
-            ws.seq = None
+            ws.seq = ws.nkeys = None
         cache.n[slot] = p0 + T
         return ws.logits[-1:].clone() if last_only else ws.logits.clone()
 
@@ -715,10 +718,11 @@ class TModel:
         ws.slot.fill_(slot)
         ws.pos.copy_(torch.arange(p0, p0 + T, dtype=I32))
         ws.seq = (slot, p0 + T) if T >= self.PREFILL_MIN_ROWS.get(self.cfg.hd, 1 << 30) else None
+        ws.nkeys = p0 + T
         try:
             self.forward_rows(ws, trace=(layout, buf), keys=p0 + T)
         finally:
-            ws.seq = None
+            ws.seq = ws.nkeys = None
         cache.n[slot] = p0 + T
         return ws.logits.clone(), layout.split(buf.cpu().numpy())
 

@@ -465,12 +465,27 @@ def qkv_rope_cache(t, s, b, cos, sin, slot, pos, cache, qq, sq, H, KV, hd, clear
               _ptr(sq), _ptr(kq), _ptr(sk), _ptr(v), R, H, KV, hd, Smax, int(clear), _stream())
 
 
-def attention(qq, sq, cache, slot, pos, expt, out, H, KV, hd, inv, obits=None):
+# A wave per (row, head) (exact_attention_rows) against a block per (row, head) (exact_attention), by the bound on the
+# positions: a wave walks its keys alone, so that few rows over many keys are faster in blocks, and blocks that run in several
+# rounds slower. us, 28 heads of 128: 4 rows to 64 keys 9.6 and 9.4, to 104 14.2 and 9.8; 24 rows to 94 14.2 and 12.3; 41 rows
+# to 41 10.1 and 14.7, to 121 19.7 and 20.3; 95 rows to 95 20.6 and 32.3. 40 heads, 20 rows to 120: 18.3 and 19.6.
+def attention_rows_keys(R, H):
+    """The largest number of positions for which attention() of R rows takes a wave per (row, head)."""
+    return 32 if R * H <= 256 else 64 if R * H <= 768 else 128
+
+
+def attention(qq, sq, cache, slot, pos, expt, out, H, KV, hd, inv, obits=None, nkeys=None):
+    """nkeys: a bound that every row's position is below, when the caller knows one."""
     R = qq.shape[0]
     kq, sk, v = cache
     Smax = kq.shape[2]
     if obits is not None:
         _need(obits, I32, "obits", R * H)
+    if nkeys is not None and 0 < nkeys <= attention_rows_keys(R, H) and hd in (64, 128) and not any(
+            a.data_ptr() % 16 for a in (qq, kq, v, out)):
+        _lib.call("exact_attention_rows", _ptr(qq), _ptr(sq), _ptr(kq), _ptr(sk), _ptr(v), _ptr(slot), _ptr(pos), _ptr(expt),
+                  _ptr(out), _ptr(obits), R, H, KV, hd, Smax, nkeys, inv, _stream())
+        return out
     _lib.call("exact_attention", _ptr(qq), _ptr(sq), _ptr(kq), _ptr(sk), _ptr(v), _ptr(slot), _ptr(pos), _ptr(expt),
               _ptr(out), _ptr(obits), R, H, KV, hd, Smax, inv, _stream())
     return out

@@ -270,3 +270,29 @@ def test_row_attention_long_context_matches_oracle():
     ops.attention(qd, sqd, cache, torch.tensor([slot], dtype=I32, device=DEV), posd,
                   torch.tensor(exp_t(), dtype=I32, device=DEV), out, H, KV, hd, O.inv_sqrt_hd(hd))
     assert np.array_equal(host(out), oracle_rows(kq, sk, v, qq, sq, pos, slot, H, KV, [0]))
+
+
+@pytest.mark.parametrize("H,KV,hd", [(7, 1, 128), (4, 4, 128), (14, 2, 64), (2, 2, 64)])
+@pytest.mark.parametrize("R,nkeys,vmag,shifts", [(1, 1, "small", 4), (5, 63, "large", 4), (9, 64, "wrap", (30, 8)),
+                                                 (41, 65, "small", 4), (95, 128, "large", 4), (128, 128, "wrap", 4),
+                                                 (3, 127, "small", 20), (64, 64, "small", (20, 16))])
+def test_short_prompt_rows_match_oracle_and_the_row_kernel(H, KV, hd, R, nkeys, vmag, shifts, monkeypatch):
+    """A wave per (row, head) (exact_attention_rows), at the edges of its 64-key chunks, in a cache longer than the prompt"""
+    monkeypatch.setattr(ops, "attention_rows_keys", lambda R, H: 128)
+    Smax, slot = nkeys + 70, 1
+    kq, sk, v, qq, sq, pos = make_case(R * 1000 + nkeys + hd, 2, slot, H, KV, hd, Smax, nkeys, R, vmag, shifts)
+    cache, dq, ds, dp = to_dev(kq, sk, v, qq, sq, pos)
+    dsl = torch.full((R,), slot, dtype=I32, device=DEV)
+    expt = torch.tensor(exp_t(), dtype=I32, device=DEV)
+    inv = O.inv_sqrt_hd(hd)
+    for table in (expt, -expt, torch.zeros_like(expt)):
+        got = []
+        for nk in (nkeys, None):
+            out = torch.full((R, H * hd), 3, dtype=I64, device=DEV)
+            ob = torch.full((R, H), -1, dtype=I32, device=DEV)
+            ops.attention(dq, ds, cache, dsl, dp, table, out, H, KV, hd, inv, ob, nkeys=nk)
+            got.append((host(out), host(ob)))
+        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+        if table is expt:
+            rows = np.arange(R)
+            assert np.array_equal(got[0][0], oracle_rows(kq, sk, v, qq, sq, pos, slot, H, KV, rows))
