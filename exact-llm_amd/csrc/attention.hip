@@ -345,7 +345,7 @@ __global__ __launch_bounds__(NT) void k_attention_qkv(const int64_t* __restrict_
   int skpre = 0;
   // KS = 8: thread (key kg = tid / 8, lane kl = tid % 8) holds dims [kl hd / 8, (kl + 1) hd / 8) of keys kg,
   // kg + NT / 8, ... (KP passes), at most 4 chunks of 16 bytes each
-  constexpr int NVC = KP > 2 ? 2 : 4;   // chunks a thread holds per key (the 4-pass variant runs at hd 128 only)
+  constexpr int NVC = KP > 2 ? 2 : 4;   // chunks a thread holds per key (more passes run at hd 64 and 128 only)
   v4i ks8[KP][NVC];
   int sks8[KP];
 #pragma unroll
@@ -972,6 +972,11 @@ extern "C" int exact_attention_qkv_split(const int64_t* t, const int32_t* s, con
   // ... and of up to 4 ATT_WIDE_THREADS / 8 positions at hd 128 in four passes
   const bool ks8_wide4 = !ks8_wide && ATT_KS8 != 0 && ATT_KS8_LONG4 != 0 && hd == 128 && hd >= ATT_KS8_WIDE_HD &&
                          Smax <= 4 * (ATT_WIDE_THREADS / 8) && blocks <= ATT_WIDE_BLOCKS;
+  // ... and at hd 64, above the narrow path's, of up to 8 ATT_THREADS / 8 positions in eight passes, where the split 4 ways
+  // fits one round (14 heads, us at 16 / 100 / 290 / 500 positions, one row: 7.06 / 7.47 / 9.12 / 10.1 against 7.35 / 7.68 /
+  // 10.5 / 13.3 of one 1024-thread block a head with a thread a key; 8 rows, split 2 ways: 7.9 against 7.2 at 16)
+  const bool ks8_hd64 = ATT_KS8 && hd == 64 && Smax > 2 * (ATT_THREADS / 8) && Smax <= 8 * (ATT_THREADS / 8) &&
+                        att_qkv_ds(obn, blocks, hd) == 4;
   const bool ks8_narrow = ATT_KS8 && hd % 64 == 0 && Smax <= 2 * (ATT_THREADS / 8);
   // blocks in several rounds (batched decode) over caches of up to 4 ATT_THREADS / 8 positions: ATT_THREADS-thread
   // blocks, 8 threads per cached key in two or four passes, exp table lookups from global memory (the LDS it would
@@ -995,6 +1000,8 @@ extern "C" int exact_attention_qkv_split(const int64_t* t, const int32_t* s, con
       att_qkv_go<ATT_MR_VPF, ATT_THREADS, ATT_KPF, 8, 2, 1, ATT_MR_GT != 0>(ATT_QKV_ARGS);
     else
       att_qkv_go<ATT_MR_VPF, ATT_THREADS, ATT_KPF, 8, 4, 1, ATT_MR_GT != 0>(ATT_QKV_ARGS);
+  } else if (ks8_hd64) {
+    att_qkv_go<8, ATT_THREADS, ATT_KPF, 8, 8, 4, ATT_GT1 != 0>(ATT_QKV_ARGS);
   } else if (ks8_wide4) {
     // value prefetch: 2 ATT_WIDE_THREADS DS / hd threads per pair cover the up to 512 positions in VPF steps
     if (ds == 4)

@@ -296,3 +296,9 @@ def test_short_prompt_rows_match_oracle_and_the_row_kernel(H, KV, hd, R, nkeys, 
         if table is expt:
             rows = np.arange(R)
             assert np.array_equal(got[0][0], oracle_rows(kq, sk, v, qq, sq, pos, slot, H, KV, rows))
+
+
+@pytest.mark.parametrize("R,Smax", [(1, 129), (1, 512), (4, 300), (2, 257)])
+def test_fused_qkv_attention_hd64_eight_passes(R, Smax):
+    """hd 64 over caches of 129 to 512 positions, four blocks a head: eight 64-key passes, 8 threads a key"""
+    test_fused_qkv_attention_matches_two_launches(14, 2, 64, R, True, Smax, 4)
