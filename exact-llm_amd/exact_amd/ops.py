@@ -7,6 +7,7 @@ registered below under the same name with the same contract: (x16 int16 (K,), wT
 Mg int64 (N, K/128)) -> int64 (N,), on the reference's own tensors with no repacking.
 """
 import ctypes
+import functools
 
 import numpy as np
 import torch
@@ -506,10 +507,15 @@ ATT_ROUND_BLOCKS = 256
 ATT_SHORT_CACHE = 512
 
 
+@functools.lru_cache(maxsize=256)
+def _attention_work_bytes(R, H, KV, hd, Smax):
+    return int(_lib.load().exact_attention_decode_workspace(R, H, KV, hd, Smax))
+
+
 def attention_keys_from(R, H, KV, hd, Smax):
     """The number of positions (keys of the longest row) from which decode attention goes split over the keys; beyond Smax
     where the split does not take the sizes."""
-    if _lib.load().exact_attention_decode_workspace(R, H, KV, hd, Smax) <= 0:
+    if _attention_work_bytes(R, H, KV, hd, Smax) <= 0:
         return Smax + 1
     if R * H <= ATT_ROUND_BLOCKS and Smax <= ATT_SHORT_CACHE:
         return Smax + 1
@@ -518,7 +524,7 @@ def attention_keys_from(R, H, KV, hd, Smax):
 
 def attention_work(R, H, KV, hd, Smax, device):
     """Workspace of one split attention_qkv call of these sizes."""
-    return torch.empty(max(1, int(_lib.load().exact_attention_decode_workspace(R, H, KV, hd, Smax))), dtype=I8, device=device)
+    return torch.empty(max(1, _attention_work_bytes(R, H, KV, hd, Smax)), dtype=I8, device=device)
 
 
 def attention_qkv(t, s, b, cos_t, sin_t, slot, pos, cache, expt, out, H, KV, hd, inv, obits=None, obn=1, keys=None, work=None):
