@@ -195,7 +195,8 @@ def _check_slot(slot, cache):
 
 class Workspace:
     """Activation buffers for R rows (allocated once; reused by every step and by captured graphs).
-    t buffers start zeroed and are left zeroed by the kernels that consume them."""
+    t buffers start zeroed; the kernels that consume them leave those zeroed that the next pass's linear may add into
+    (TModel._adds), and the others as they are."""
 
     def __init__(self, cfg, R, device, nq, I, abits=15):
         D, H, hd, V = cfg.D, cfg.H, cfg.hd, cfg.V
@@ -313,8 +314,8 @@ class TModel:
 
     # ---------------------------------------------------------------- linears
     def _lin(self, x, lin, out, x8=None):
-        """t for a group-mode linear (the consumer kernel applies shr(t, 28 - s) + b and leaves out zeroed,
-        so decode-sized calls accumulate into it without a separate clear). x8: x's digit rows, when its producer
+        """t for a group-mode linear (the consumer kernel applies shr(t, 28 - s) + b and leaves out zeroed
+        where the call adds into it, so that no call needs a separate clear). x8: x's digit rows, when its producer
         wrote them."""
         return ops.linear_t(x, self.abits, lin, out, zeroed=True, x8=x8)
 
