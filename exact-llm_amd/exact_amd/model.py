@@ -405,9 +405,9 @@ class TModel:
         # one per CU)
         fsfuse = (self.FFN_NORM and sfuse and qfuse and D > ops.NORM_SWIGLU_KMAX and D <= ops.NORM_SWIGLU_WIDE_KMAX
                   and c.I % 128 == 0)
-        # prompts whose gate|up GEMM splits no K: the SwiGLU in its epilogue (no totals in memory, no SwiGLU launch)
-        gsfuse = (group and not keep and not c.moe and self.abits == 15 and R > ops.A16_DIGIT_ROWS
-                  and ops.gemm_swiglu_supported(R, self.w.layers[0]["gateup"]))
+        # prompts whose gate|up GEMM splits no K: the SwiGLU in its epilogue (no totals in memory, no SwiGLU launch), in the
+        # layers whose linear it takes (a layer of wide scales writes its totals, all of them, as it splits no K either)
+        gsfuse = group and not keep and not c.moe and self.abits == 15 and R > ops.A16_DIGIT_ROWS
         if ws.h is None and not c.moe and ((xfuse and (c.I > 8192 or nfuse or sfuse)) or sqfuse):
             ws.h = torch.zeros((R, ws.I), dtype=I64, device=self.dev)
         x_cur, x_nxt = ws.x, ws.x2
@@ -516,7 +516,7 @@ class TModel:
                 ops.quant_rows(ws.h, ws.part_sw, c.I // ops.SWIGLU_PART_COLS, self.abits, ws.hq, ws.sh, x8=dh)
                 self._lin(ws.hq, L["down"], t_d, x8=dh)
                 res_t, res_s = t_d, ws.sh
-            elif gsfuse:   # h takes the place of the totals, which this workspace then never holds
+            elif gsfuse and ops.gemm_swiglu_supported(R, L["gateup"]):   # h takes the place of the totals, which this workspace then never holds
                 ops.gemm_swiglu_qrow(dx, L["gateup"], ws.s, tab.silu, t_gu, ws.part_sw, ws.hq, ws.sh, dh)
                 self._lin(ws.hq, L["down"], t_d, x8=dh)
                 res_t, res_s = t_d, ws.sh

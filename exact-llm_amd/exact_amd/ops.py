@@ -419,6 +419,8 @@ def gemm_swiglu_qrow(x8, lin, s, silu, h, part, xq, sq, xq8=None):
     xq (int16), sq and the digit rows xq8: the results of swiglu_qrow on the linear's totals. h: (R, I) int64 and part:
     (R, I / 32) int32 scratch."""
     R, I = s.numel(), lin.N // 2
+    if lin.mh is not None or lin.bias is not None:
+        raise ExactError("gemm_swiglu_qrow: linears with wide scales or a bias take gemm_g128 and swiglu_qrow")
     _need_packed(lin, "gemm_swiglu_qrow")
     _lib.call("exact_gemm_g128_digits_swiglu", _digits(x8, R, lin.K), _ptr(lin.wp), _ptr(lin.mp), _ptr(colterm(lin)),
               _ptr(_need(s, I32, "s", R)), _ptr(silu), _ptr(_need(h, I64, "h", R * I)),

@@ -9,6 +9,7 @@ import torch
 import exact_oracle as O
 from exact_amd import artifact
 from exact_amd import convert as C
+from exact_amd import ops, synth
 from exact_amd.model import DeviceWeights, TModel
 from test_convert_cpu import fake_checkpoint, oracle_arrays
 
@@ -55,3 +56,29 @@ def test_converted_checkpoint_matches_oracle(tmp_path, mode, tie):
         lg, nid = tm2.decode_rows([tok], cache)
         assert np.array_equal(host(lg)[0], orows[i]), i
         tok = int(host(nid)[0])
+
+
+@pytest.mark.parametrize("wide", [0, 1])
+@pytest.mark.parametrize("T", [70, 200, 300])
+def test_wide_scales_in_one_layer_only(wide, T):
+    """Which planes a linear has is its own affair: gate|up scales past int16 in one layer and within it in the other, with
+    prompts below and on the sizes whose narrow layers take the SwiGLU in the GEMM's epilogue"""
+    cfg = synth.CONFIGS["tiny"]
+    rng = np.random.default_rng(10 * T + wide)
+    arr = dict(emb=rng.integers(-(1 << 16), 1 << 16, (cfg.V, cfg.D)), gf=rng.integers(60000, 70000, cfg.D))
+    shapes = dict(q=(cfg.D, cfg.H * cfg.hd), k=(cfg.D, cfg.KV * cfg.hd), v=(cfg.D, cfg.KV * cfg.hd), o=(cfg.H * cfg.hd, cfg.D),
+                  gate=(cfg.D, cfg.I), up=(cfg.D, cfg.I), down=(cfg.I, cfg.D))
+    for i in range(cfg.NL):
+        arr[f"{i}.g1"], arr[f"{i}.g2"] = rng.integers(60000, 70000, (2, cfg.D))
+        for n, (K, N) in shapes.items():
+            arr[f"{i}.{n}.w"] = rng.integers(-127, 128, (K, N)).astype(np.int8)
+            M = rng.integers(synth.M_LO, synth.M_HI, (K // 128, N))
+            arr[f"{i}.{n}.M"] = M + (rng.integers(0, 3, M.shape) << 15 if i == wide and n in ("gate", "up") else 0)
+    arr["head.w"] = rng.integers(-127, 128, (cfg.D, cfg.V)).astype(np.int8)
+    arr["head.M"] = rng.integers(1 << 12, 1 << 14, cfg.V)
+    tm = TModel(DeviceWeights.from_arrays(cfg, arr, DEV), Smax=T + 4)
+    assert [L["gateup"].mh is not None for L in tm.w.layers] == [i == wide for i in range(cfg.NL)]
+    assert ops.gemm_swiglu_supported(T, tm.w.layers[1 - wide]["gateup"]) == (T > 150)
+    ids = rng.integers(0, cfg.V, T).tolist()
+    cache = tm.new_cache(B=1)
+    assert np.array_equal(host(tm.forward(ids, cache)), oracle_model(arr, cfg, "group", T + 4)(ids))

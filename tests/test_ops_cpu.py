@@ -26,3 +26,16 @@ def test_norm_gemv_one_block_per_cu_reads_the_kernel_split():
     assert ops.norm_gemv_one_block_per_cu(4608, 3584, R=2, cus=256)
     assert not ops.norm_gemv_one_block_per_cu(4608, 3584, R=3, cus=256)      # the launch takes at most 2 rows
     assert _lib.load().exact_gemv_g128_norm_acc_blockwaves(1, 4608, 100, 256) == 0   # K % 128: refused
+
+
+def test_swiglu_gemm_refuses_wide_scales_and_biases():
+    """gemm_swiglu_qrow hands the kernel the low scale plane and no bias, so a linear with either more is refused (before any
+    buffer is looked at), and gemm_swiglu_supported says so"""
+    import torch
+    from exact_amd import ops
+    wp, mp = torch.zeros(4 * 2 * 8192, dtype=torch.int8), torch.ones(4 * 2 * 64, dtype=torch.int16)
+    for kw in (dict(mh=torch.ones_like(mp)), dict(bias=torch.zeros(256, dtype=torch.int64))):
+        lin = ops.PackedLinear(wp, mp, 256, 256, **kw)
+        assert not ops.gemm_swiglu_supported(512, lin)
+        with pytest.raises(_lib.ExactError, match="wide scales or a bias"):
+            ops.gemm_swiglu_qrow(None, lin, torch.zeros(512, dtype=torch.int32), None, None, None, None, None)
