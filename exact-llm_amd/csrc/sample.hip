@@ -101,9 +101,10 @@ __host__ __forceinline__ SampleWork sample_work(int64_t* w, int64_t n, int64_t R
 }
 
 // floor(e * 2^20 / es), rb ~ 2^20 / es: for 0 <= e <= es the quotient is at most 2^20 and the float64 estimate within one
-// of it; anything else (an exp table with negative entries) takes the general division
+// of it; anything else (an exp table with negative entries, or one that leaves a row no exponential) takes the general
+// division, which gives 0 for es <= 0
 __device__ __forceinline__ int64_t sample_p(int32_t e, int64_t es, double rb) {
-  if (e < 0 || e > es) return floordiv_pos(shl64(e, 20), es);
+  if (e < 0 || e > es || es <= 0) return floordiv_pos(shl64(e, 20), es);
   uint32_t q = (uint32_t)((double)e * rb);
   const int64_t d = ((int64_t)e << 20) - (int64_t)q * es;
   return (int64_t)q + (d >= es) - (d < 0);

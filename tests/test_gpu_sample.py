@@ -118,3 +118,26 @@ def test_split_rows_of_a_table_with_negative_entries_match_the_one_block_kernel(
         out.append((host(ids), host(pd)))
     assert (out[0][1] < 0).any()
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("table", ["zeros", "zero sum"])
+def test_split_rows_of_no_exponential_match_the_one_block_kernel(table):
+    """a softmax denominator of 0, from a table of zeros and from entries that cancel: every p is 0 and so is every prefix
+    sum, so that the token is V"""
+    V, R, seed, tnum = 5000, 3, 11, ops.temp_num(1.0)
+    tab = np.zeros_like(np.array(exp_t(), dtype=np.int64))
+    lg = torch.zeros((R, V), dtype=I64, device=DEV)
+    if table == "zero sum":   # 2000 logits each of 1000 and of -1000, 1 below the maximum, and 1000 of 0, 2 below it
+        tab[0], tab[256:258] = 1000, -1000
+        lg[:, ::2] = -(1 << 16)
+        lg[:, ::5] = -(2 << 16)
+    expt = torch.tensor(tab, dtype=I32, device=DEV)
+    step = torch.arange(R, dtype=I32, device=DEV)
+    for lim in (V + 1, 1):
+        ids, pd = torch.zeros(R, dtype=I32, device=DEV), torch.full((R, V), 7, dtype=I64, device=DEV)
+        old, ops.SAMPLE_SPLIT_FROM = ops.SAMPLE_SPLIT_FROM, lim
+        try:
+            ops.sample(lg, seed, step, tnum, expt, ids, pd)
+        finally:
+            ops.SAMPLE_SPLIT_FROM = old
+        assert (host(ids) == V).all() and not host(pd).any(), lim
