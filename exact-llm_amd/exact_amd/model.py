@@ -900,13 +900,15 @@ class GraphDecoder:
 
     def capture(self):
         """Warm up once outside the graph (restoring positions), then capture one step (one per trace buffer, and one more
-        each for the attention split over the keys where the positions can still grow into it)."""
+        each for the attention split over the keys where the cache is long enough for it), in place of what an earlier call
+        captured: a decoder serves sequences after the one that it was captured with, shorter ones among them."""
         ws = self.ws
+        self.graph, self.graphs = None, {}
         pos0 = ws.pos.clone()
         ids0 = ws.ids.clone()
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
-        modes = [True] if self._split() else [False] + [True] * (self.keys_from <= self.tm.Smax)
+        modes = [False] + [True] * (self.keys_from <= self.tm.Smax)
         if True in modes:
             self.tm.attention_work(ws)   # on this stream, as the workspace's other buffers
         with torch.cuda.stream(s):
@@ -939,8 +941,7 @@ class GraphDecoder:
         if not self.graphs:
             self._step(b)
         else:
-            split = self._split() or (False, 0) not in self.graphs   # the same results from either
-            self.graphs[split, b if self.trace else 0].replay()
+            self.graphs[self._split(), b if self.trace else 0].replay()
         if self.recorder is not None:
             self.recorder.after_step(b)
         self.nstep += 1

@@ -134,3 +134,36 @@ def test_grouped_batch_attention_of_eight_heads():
     ops.attention(qq, sq, c_a, slot, pos, expt, out_a, H, KV, hd, inv)
     ops.attention_qkv(t, s, None, cos, sin, slot, pos, c_b, expt, out_b, H, KV, hd, inv, obn=4, keys=1)
     assert torch.equal(out_a, out_b) and all(torch.equal(x, y) for x, y in zip(c_a, c_b))
+
+
+def test_captured_again_for_another_cache_over_the_line(monkeypatch):
+    """A decoder captured below the position from which attention is split, then again with another cache above it: every
+    later step, short positions among them, reads and writes that cache, and short positions keep the one launch"""
+    from exact_amd.model import DeviceWeights, GraphDecoder, TModel
+    monkeypatch.setattr(ops, "ATT_SHORT_CACHE", 0)
+    monkeypatch.setattr(ops, "ATT_KEYS_WORK", 50 * 128)
+    cfg = synth.CONFIGS["tiny-hd128"]
+    tm = TModel(DeviceWeights.synthetic(cfg, 3, DEV), Smax=96)
+    prompt = lambda n: [(11 * i + 3) % cfg.V for i in range(n)]
+    want, ref = [], tm.new_cache()
+    for n in (60, 20):
+        ref.n[0] = 0
+        tm.forward(prompt(n), ref, last_only=True)
+        want.append([x.clone() for x in tm.decode_rows([5], ref)])
+    first, cache = tm.new_cache(), tm.new_cache()
+    tm.forward(prompt(12), first, last_only=True)
+    gd = GraphDecoder(tm, first, 1)
+    gd.load([5])
+    gd.capture()
+    old = [[x.clone() for x in layer] for layer in first.layers]
+    gd.cache = cache
+    for i, n in enumerate((60, 20)):
+        cache.n[0] = 0
+        tm.forward(prompt(n), cache, last_only=True)
+        gd.load([5])
+        if i == 0:
+            gd.capture()
+        assert gd._split() == (n == 60) and set(gd.graphs) == {(False, 0), (True, 0)}
+        assert all(torch.equal(x, y) for x, y in zip(gd.step(), want[i])), n
+    assert all(torch.equal(x, y) for a, b in zip(old, first.layers) for x, y in zip(a, b))
+    assert all(torch.equal(x[:, :, :21], y[:, :, :21]) for a, b in zip(cache.layers, ref.layers) for x, y in zip(a, b))
