@@ -498,13 +498,19 @@ ATT_SPLIT_MAX = 4   # bit lengths a head that attention_qkv may write (blocks a 
 
 
 # Decode attention split over the keys (exact_attention_decode, four launches) against one launch with a block per (row,
-# head), whose time grows with the positions: in a graph, us a layer at 17 / 301 / 601 / 6002 positions, one row of 28 heads
-# over 4 KV heads of 128: 8.0 / 15.3 / 24.2 / 182 in one launch, 15.2 / 16.3 / 17.2 / 21.4 split. Heads of 64 halve the slope
-# (401 positions: 10.3 and 13.5), and caches of at most 512 positions have faster one-launch variants (401 positions of 512:
-# 11.3 and 16.1). Where the (row, head) blocks run in several rounds (8 rows of 40 heads over 8) the lines meet earlier:
-# 16.8 in two launches and 18.0 split at 131 positions, 239 and 67 at 3001.
-ATT_KEYS_WORK = 384 * 128
-ATT_KEYS_WORK_ROUNDS = 192 * 128
+# head), whose time grows with the positions. In a graph, us a layer at 17 / 301 / 601 / 6002 positions, one row of 28 heads
+# over 4 KV heads of 128: 8.0 / 15.3 / 24.2 / 182 in one launch, 15.2 / 16.3 / 17.2 / 21.4 split; they meet at 360. Heads of 64
+# halve the slope (401 positions: 10.3 and 13.5), and caches of at most 512 positions have faster one-launch variants (401
+# positions of 512: 11.3 and 16.1). Where the (row, head) blocks run in several rounds (8 rows of 40 heads over 8) the lines
+# meet earlier: 17.6 in two launches and 17.8 split at 150 of 300 positions.
+# The split's grids cover the cache, ceil(Smax / 128) blocks a (row, KV head), as a graph's launches serve every position: the
+# blocks past a row's position leave at once, but not for nothing. 8 rows of 40 heads over 8, at 200 positions of 300 / 1024 /
+# 4096 (192 / 512 / 2048 blocks): 18.4 / 24.9 / 52 us; 8 rows of 16 heads over 16, at 384 positions of 1024 / 4096 (1024 / 4096
+# blocks): 34 / 73 against 27 and 28 in one launch, and the lines meet at 600 / 1400 positions. So the line moves up by about 0.4
+# positions a block past the first 160 (0.2 in several rounds).
+ATT_KEYS_WORK, ATT_BLOCK_WORK = 384 * 128, 51
+ATT_KEYS_WORK_ROUNDS, ATT_BLOCK_WORK_ROUNDS = 192 * 128, 25
+ATT_FREE_BLOCKS = 160
 ATT_ROUND_BLOCKS = 256
 ATT_SHORT_CACHE = 512
 
@@ -521,7 +527,9 @@ def attention_keys_from(R, H, KV, hd, Smax):
         return Smax + 1
     if R * H <= ATT_ROUND_BLOCKS and Smax <= ATT_SHORT_CACHE:
         return Smax + 1
-    return (ATT_KEYS_WORK if R * H <= ATT_ROUND_BLOCKS else ATT_KEYS_WORK_ROUNDS) // hd + 1
+    work, per = ((ATT_KEYS_WORK, ATT_BLOCK_WORK) if R * H <= ATT_ROUND_BLOCKS else
+                 (ATT_KEYS_WORK_ROUNDS, ATT_BLOCK_WORK_ROUNDS))
+    return (work + per * max(R * KV * -(-Smax // 128) - ATT_FREE_BLOCKS, 0)) // hd + 1
 
 
 def attention_work(R, H, KV, hd, Smax, device):

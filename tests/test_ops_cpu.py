@@ -39,3 +39,23 @@ def test_swiglu_gemm_refuses_wide_scales_and_biases():
         assert not ops.gemm_swiglu_supported(512, lin)
         with pytest.raises(_lib.ExactError, match="wide scales or a bias"):
             ops.gemm_swiglu_qrow(None, lin, torch.zeros(512, dtype=torch.int32), None, None, None, None, None)
+
+
+# us a layer in a graph, (heads, KV heads, hd), rows, cache length, position: one launch (two where rows x heads pass 256 and the
+# cache 256 positions) and split over the keys
+ATT_TIMES = [((16, 16, 128), 8, 4096, 384, 27.7, 72.6), ((16, 16, 128), 8, 8192, 512, 34.6, 78.1),
+             ((16, 16, 128), 16, 4096, 1024, 74.2, 138.1), ((40, 8, 128), 8, 4096, 256, 30.6, 53.0),
+             ((40, 8, 128), 16, 4096, 640, 71.9, 95.3), ((28, 4, 128), 8, 8192, 512, 26.6, 37.7),
+             ((28, 4, 128), 1, 8192, 300, 15.7, 17.1), ((14, 2, 64), 8, 8192, 768, 18.2, 22.3),
+             ((28, 4, 128), 1, 8192, 640, 25.4, 17.5), ((28, 4, 128), 8, 1024, 512, 26.7, 21.4),
+             ((28, 4, 128), 8, 4096, 1024, 47.2, 36.6), ((40, 8, 128), 8, 1024, 320, 34.1, 25.6),
+             ((40, 8, 128), 16, 2048, 768, 83.5, 58.8), ((16, 16, 128), 1, 4096, 640, 26.3, 18.5),
+             ((16, 16, 128), 8, 1024, 768, 47.0, 39.5), ((14, 2, 64), 1, 4096, 1024, 21.5, 13.9)]
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
+@pytest.mark.parametrize("heads,R,Smax,pos,one,split", ATT_TIMES)
+def test_attention_split_line_against_measured_times(heads, R, Smax, pos, one, split):
+    """the faster of the two paths, at times measured well off the line: caches much longer than their positions too"""
+    from exact_amd import ops
+    assert (pos + 1 >= ops.attention_keys_from(R, *heads, Smax)) == (split < one)
