@@ -268,7 +268,7 @@ class TModel:
         self.nl = len(weights.layers)
         self.nq = (c.H + 2 * c.KV) * c.hd
         self.I = c.I if not c.moe else 1
-        self._ws, self._adds_R = {}, {}
+        self._ws, self._adds_R, self._eager_from = {}, {}, {}
         self._pws = None
         self._graphs = collections.OrderedDict()   # captured prefill passes
 
@@ -300,6 +300,14 @@ class TModel:
         if self._pws is None or self._pws[0] < R:
             self._pws = (R, ops.prefill_workspace(R, self.cfg.H, self.cfg.KV, self.cfg.hd, self.Smax, self.dev))
         return self._pws[1]
+
+    def eager_keys_from(self, R):
+        """Positions from which decode attention of R rows is split over the keys in a pass outside a graph."""
+        c = self.cfg
+        if R not in self._eager_from:
+            nbytes = sum(lin.wp.numel() for lin in self.w.layers[0].values() if isinstance(lin, PackedLinear)) if self.nl else 0
+            self._eager_from[R] = ops.attention_eager_keys_from(R, c.H, c.KV, c.hd, self.Smax, nbytes)
+        return self._eager_from[R]
 
     def attention_work(self, ws):
         if ws.att_work is None:
@@ -334,14 +342,14 @@ class TModel:
         return self._adds_R[R]
 
     # ---------------------------------------------------------------- one pass over R rows
-    def forward_rows(self, ws, want_logits=True, trace=None, independent=False, last_only=False, keys=None):
+    def forward_rows(self, ws, want_logits=True, trace=None, independent=False, last_only=False, keys=None, split=None):
         """Runs the model on ws.ids with (slot, pos) per row; KV of each row is written into the cache
         at (slot, pos). Leaves logits in ws.logits and greedy ids in ws.next_ids (last_only: of the last row only, the
         others are left as they were; the final norm, the head and the argmax run on that row alone).
         independent: every row is a different sequence (decode), so no row attends to another row's new key and
         the q/k/v epilogue runs inside the attention launch.
-        keys: the positions the pass's longest row attends to, when the caller knows them (else the cache's): they decide
-        whether decode attention is split over the keys.
+        keys: the positions the pass's longest row attends to, when the caller knows them: they decide whether decode
+        attention is split over the keys, unless split says so (a pass under capture, whose positions will grow).
         trace: (TraceLayout, int64 device buffer): every linear's totals t are produced in the buffer's slots
         and left there (the buffer is zeroed first); the consumer kernels read them without clearing."""
         c, R, tab = self.cfg, ws.R, self.tab
@@ -368,9 +376,9 @@ class TModel:
         xfuse = group and R <= self.QROW_FUSE_ROWS
         afuse = xfuse and ws.seq is None and (R == 1 or independent)
         # decode attention over many positions: split over the keys, the q|k|v epilogue inside at any batch
-        keys = min(keys or self.Smax, self.Smax)
-        ksplit = (group and ws.seq is None and (R == 1 or independent)
-                  and keys >= ops.attention_keys_from(R, H, KV, hd, self.Smax))
+        if split is None:
+            split = min(keys or self.Smax, self.Smax) >= self.eager_keys_from(R)
+        ksplit = split and group and ws.seq is None and (R == 1 or independent)
         if ksplit:
             self.attention_work(ws)
         # batched decode rows (each its own sequence): the q|k|v epilogue inside the attention launch as well, whose
@@ -447,7 +455,8 @@ class TModel:
             nob = H   # bit lengths per row that attention leaves in ws.obits
             if afuse or bfuse:
                 ops.attention_qkv(t_qkv, s_qkv, b_qkv, tab.cos, tab.sin, ws.slot, ws.pos, cache, tab.exp, ws.att, H, KV, hd,
-                                  tab.inv, ws.obits, obn=self.ATT_SPLIT, keys=keys, work=ws.att_work)
+                                  tab.inv, ws.obits, obn=self.ATT_SPLIT, keys=self.Smax if ksplit else 1,
+                                  work=ws.att_work if ksplit else None)
                 nob = H * self.ATT_SPLIT
             else:
                 ops.qkv_rope_cache(t_qkv if group else ws.t_qkv, s_qkv, b_qkv, tab.cos, tab.sin, ws.slot, ws.pos, cache,
@@ -893,9 +902,8 @@ class GraphDecoder:
 
     def _step(self, b=0, split=None):
         self.tm._cache = self.cache
-        split = self._split() if split is None else split
         self.tm.forward_rows(self.ws, trace=(self.layout, self.trace_bufs[b]) if self.trace else None, independent=True,
-                             keys=self.tm.Smax if split else 1)
+                             keys=max(self.cache.n[:self.B]) + 1, split=split)
         ops.advance(self.ws.pos)
 
     def capture(self):

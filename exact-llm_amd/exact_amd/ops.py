@@ -532,6 +532,22 @@ def attention_keys_from(R, H, KV, hd, Smax):
     return (work + per * max(R * KV * -(-Smax // 128) - ATT_FREE_BLOCKS, 0)) // hd + 1
 
 
+# ... and the positions of hd 128 below which a whole pass that the host launches kernel by kernel is not split, in one round
+# of blocks and in several, for layers of fewer than ATT_EAGER_BYTES of weights and for larger ones. The three more launches
+# cost the host 8 us a layer, which the pass hides only while the device is the slower of the two: a layer takes the host
+# about 75 us (a mixture's 135 or more). us a pass of 8 layers and the head, one launch and split: 7B shape (233 MB a layer) 776 /
+# 782 at 384 positions, 866 / 786 at 768; 0.5B shape (15 MB) 597 / 671 at 1000 and 599 / 664 at 1500, of 2048; mixture of 2.7B
+# active (52 MB) 1076 / 1149 at 768. So a small layer is split where its attention alone takes the host's time.
+ATT_EAGER_BYTES = 128 << 20
+ATT_EAGER_KEYS = {False: (2304, 768), True: (512, 256)}
+
+
+def attention_eager_keys_from(R, H, KV, hd, Smax, layer_bytes):
+    """attention_keys_from() for a pass over layers of layer_bytes of weights that runs outside a graph."""
+    least = ATT_EAGER_KEYS[layer_bytes >= ATT_EAGER_BYTES][R * H > ATT_ROUND_BLOCKS] * 128 // hd
+    return max(attention_keys_from(R, H, KV, hd, Smax), least + 1)
+
+
 def attention_work(R, H, KV, hd, Smax, device):
     """Workspace of one split attention_qkv call of these sizes."""
     return torch.empty(max(1, _attention_work_bytes(R, H, KV, hd, Smax)), dtype=I8, device=device)

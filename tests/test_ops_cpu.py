@@ -59,3 +59,18 @@ def test_attention_split_line_against_measured_times(heads, R, Smax, pos, one, s
     """the faster of the two paths, at times measured well off the line: caches much longer than their positions too"""
     from exact_amd import ops
     assert (pos + 1 >= ops.attention_keys_from(R, *heads, Smax)) == (split < one)
+
+
+# us a pass of 8 layers and the head launched by the host, (heads, KV heads, hd), MB a layer, rows, position (of 2048)
+ATT_EAGER_TIMES = [((14, 2, 64), 15, 1, 1000, 597, 671), ((14, 2, 64), 15, 1, 1500, 599, 664), ((14, 2, 64), 15, 8, 1500, 836, 901),
+                   ((16, 16, 128), 52, 1, 768, 1076, 1149), ((16, 16, 128), 52, 8, 768, 1518, 1578),
+                   ((28, 4, 128), 233, 1, 200, 737, 786), ((28, 4, 128), 233, 1, 768, 866, 786),
+                   ((28, 4, 128), 233, 8, 384, 1034, 1074), ((28, 4, 128), 233, 8, 1000, 1238, 1088)]
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
+@pytest.mark.parametrize("heads,MB,R,pos,one,split", ATT_EAGER_TIMES)
+def test_attention_split_line_of_eager_passes_against_measured_times(heads, MB, R, pos, one, split):
+    """a pass that the host's launches bound keeps the one launch a layer"""
+    from exact_amd import ops
+    assert (pos + 1 >= ops.attention_eager_keys_from(R, *heads, 2048, MB * 10**6)) == (split < one)
