@@ -377,7 +377,7 @@ class TModel:
         afuse = xfuse and ws.seq is None and (R == 1 or independent)
         # decode attention over many positions: split over the keys, the q|k|v epilogue inside at any batch
         if split is None:
-            split = min(keys or self.Smax, self.Smax) >= self.eager_keys_from(R)
+            split = ops.known_keys(keys, self.Smax) >= self.eager_keys_from(R)
         ksplit = split and group and ws.seq is None and (R == 1 or independent)
         if ksplit:
             self.attention_work(ws)

@@ -548,6 +548,14 @@ def attention_eager_keys_from(R, H, KV, hd, Smax, layer_bytes):
     return max(attention_keys_from(R, H, KV, hd, Smax), least + 1)
 
 
+def known_keys(keys, Smax):
+    """The longest row's positions as the lines take them. A caller that does not tell (keys None) may be anywhere in its cache,
+    so the middle stands for them: averaged over the positions of a cache, the split is the faster one from just about the
+    caches whose middle is past the line. us a call launched by the host, one row of 28 heads over 4, averages of one launch and
+    split: 15.2 and 19.5 at 520 positions of cache, 22.5 and 19.6 at 1024; at 17 positions 11.5 and 18.6, at 600 23.7 and 18.5."""
+    return min(keys, Smax) if keys else (Smax + 1) // 2
+
+
 def attention_work(R, H, KV, hd, Smax, device):
     """Workspace of one split attention_qkv call of these sizes."""
     return torch.empty(max(1, _attention_work_bytes(R, H, KV, hd, Smax)), dtype=I8, device=device)
@@ -556,9 +564,10 @@ def attention_work(R, H, KV, hd, Smax, device):
 def attention_qkv(t, s, b, cos_t, sin_t, slot, pos, cache, expt, out, H, KV, hd, inv, obits=None, obn=1, keys=None, work=None):
     """qkv_rope_cache + attention for rows that each own their (slot, position); t unchanged.
     obits (optional) gets obn entries per head (1, 2 or ATT_SPLIT_MAX; their max is the head's bit length): with obn > 1
-    the library may split each head's p.V over obn blocks, one output slice each. keys: the longest row's positions when
-    the caller knows them (else the cache's): from attention_keys_from() on the call is split over the keys (work: its
-    attention_work(), else allocated here), and one launch below. The results are the same either way."""
+    the library may split each head's p.V over obn blocks, one output slice each. keys: the longest row's positions, which a
+    caller with short rows in a long cache does well to tell (else half of the cache's): from attention_keys_from() on the call
+    is split over the keys (work: its attention_work(), else allocated here), and one launch below. The results are the same
+    either way."""
     R = t.shape[0]
     kq, sk, v = cache
     _need(t, I64, "t", R * (H + 2 * KV) * hd)
@@ -568,7 +577,7 @@ def attention_qkv(t, s, b, cos_t, sin_t, slot, pos, cache, expt, out, H, KV, hd,
     args = (_ptr(t), _ptr(_need(s, I32, "s", R)), _ptr(b), _ptr(cos_t), _ptr(sin_t), _ptr(slot), _ptr(pos), _ptr(kq),
             _ptr(sk), _ptr(v), _ptr(expt), _ptr(out), _ptr(obits))
     Smax = kq.shape[2]
-    if min(keys or Smax, Smax) >= attention_keys_from(R, H, KV, hd, Smax) and expt.data_ptr() % 16 == 0:
+    if known_keys(keys, Smax) >= attention_keys_from(R, H, KV, hd, Smax) and expt.data_ptr() % 16 == 0:
         work = attention_work(R, H, KV, hd, Smax, t.device) if work is None else work
         _lib.call("exact_attention_decode", *args, obn, _ptr(_need(work, I8, "work")), work.numel(), R, H, KV, hd, Smax, inv,
                   _stream())

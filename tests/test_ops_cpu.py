@@ -74,3 +74,19 @@ def test_attention_split_line_of_eager_passes_against_measured_times(heads, MB, 
     """a pass that the host's launches bound keeps the one launch a layer"""
     from exact_amd import ops
     assert (pos + 1 >= ops.attention_eager_keys_from(R, *heads, 2048, MB * 10**6)) == (split < one)
+
+
+# us a call in a graph averaged over the positions of a cache, (heads, KV heads, hd), rows, cache length: one launch and split
+ATT_MEANS = [((28, 4, 128), 1, 520, 14.6, 16.4), ((28, 4, 128), 1, 1024, 22.3, 17.8), ((28, 4, 128), 8, 520, 14.4, 18.6),
+             ((28, 4, 128), 8, 4096, 88.2, 40.0), ((14, 2, 64), 8, 1024, 13.8, 14.9), ((14, 2, 64), 8, 4096, 48.1, 22.2),
+             ((16, 16, 128), 8, 1024, 33.5, 35.9), ((16, 16, 128), 16, 4096, 138.4, 169.3), ((16, 16, 128), 2, 4096, 114.7, 29.6),
+             ((40, 8, 128), 8, 1024, 58.7, 26.2)]
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
+@pytest.mark.parametrize("heads,R,Smax,one,split", ATT_MEANS)
+def test_attention_without_known_positions_takes_the_faster_path_on_average(heads, R, Smax, one, split):
+    """attention_qkv without keys: rows anywhere in the cache"""
+    from exact_amd import ops
+    assert (ops.known_keys(None, Smax) >= ops.attention_keys_from(R, *heads, Smax)) == (split < one)
+    assert ops.known_keys(Smax + 9, Smax) == Smax and ops.known_keys(7, Smax) == 7
