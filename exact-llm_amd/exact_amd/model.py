@@ -227,7 +227,7 @@ class Workspace:
         self.nkeys = None   # ... and a bound on the rows' positions
         self.h = None     # (R, I) SwiGLU values when the gate|up totals must stay intact (trace capture)
         self.hsh = None   # (R, SI) SwiGLU values of the MoE shared expert (decode rows)
-        self.att_work = None   # of decode attention split over the keys
+        self.att_work = {}     # of decode attention split over the keys: cache length -> buffer (captured graphs hold them)
         self.eh = self.part_eh = None   # the routed experts' SwiGLU values per pair and their slice bit lengths
         self.I = I
         # int16 GEMM rows (prefill above 16 rows): the producers also write their rows' int8 digit rows, which the
@@ -309,11 +309,12 @@ class TModel:
             self._eager_from[R] = ops.attention_eager_keys_from(R, c.H, c.KV, c.hd, self.Smax, nbytes)
         return self._eager_from[R]
 
-    def attention_work(self, ws):
-        if ws.att_work is None:
+    def attention_work(self, ws, Smax):
+        """Workspace of the split attention of ws's rows over a cache of Smax positions, which may be longer than the model's."""
+        if Smax not in ws.att_work:
             c = self.cfg
-            ws.att_work = ops.attention_work(ws.R, c.H, c.KV, c.hd, self.Smax, self.dev)
-        return ws.att_work
+            ws.att_work[Smax] = ops.attention_work(ws.R, c.H, c.KV, c.hd, Smax, self.dev)
+        return ws.att_work[Smax]
 
     def workspace(self, R):
         if R not in self._ws:
@@ -379,8 +380,7 @@ class TModel:
         if split is None:
             split = ops.known_keys(keys, self.Smax) >= self.eager_keys_from(R)
         ksplit = split and group and ws.seq is None and (R == 1 or independent)
-        if ksplit:
-            self.attention_work(ws)
+        att_work = self.attention_work(ws, self._cache.Smax) if ksplit else None
         # batched decode rows (each its own sequence): the q|k|v epilogue inside the attention launch as well, whose
         # totals the attention output's qrow launch then clears (caches of up to 256 positions: 8 threads per key; longer
         # ones while the (row, head) blocks fit one round: 8 rows of 28 heads at 301 positions 14.4 against 21.1 us)
@@ -455,8 +455,7 @@ class TModel:
             nob = H   # bit lengths per row that attention leaves in ws.obits
             if afuse or bfuse:
                 ops.attention_qkv(t_qkv, s_qkv, b_qkv, tab.cos, tab.sin, ws.slot, ws.pos, cache, tab.exp, ws.att, H, KV, hd,
-                                  tab.inv, ws.obits, obn=self.ATT_SPLIT, keys=self.Smax if ksplit else 1,
-                                  work=ws.att_work if ksplit else None)
+                                  tab.inv, ws.obits, obn=self.ATT_SPLIT, keys=self.Smax if ksplit else 1, work=att_work)
                 nob = H * self.ATT_SPLIT
             else:
                 ops.qkv_rope_cache(t_qkv if group else ws.t_qkv, s_qkv, b_qkv, tab.cos, tab.sin, ws.slot, ws.pos, cache,
@@ -918,7 +917,7 @@ class GraphDecoder:
         s.wait_stream(torch.cuda.current_stream())
         modes = [False] + [True] * (self.keys_from <= self.tm.Smax)
         if True in modes:
-            self.tm.attention_work(ws)   # on this stream, as the workspace's other buffers
+            self.tm.attention_work(ws, self.cache.Smax)   # on this stream, as the workspace's other buffers
         with torch.cuda.stream(s):
             for m in modes:
                 self._step(split=m)

@@ -167,3 +167,34 @@ def test_captured_again_for_another_cache_over_the_line(monkeypatch):
         assert all(torch.equal(x, y) for x, y in zip(gd.step(), want[i])), n
     assert all(torch.equal(x, y) for a, b in zip(old, first.layers) for x, y in zip(a, b))
     assert all(torch.equal(x[:, :, :21], y[:, :, :21]) for a, b in zip(cache.layers, ref.layers) for x, y in zip(a, b))
+
+
+def test_cache_longer_than_the_model(monkeypatch):
+    """A cache made for more positions than the model's own: the split's workspace goes by the cache, before and after one of
+    the model's length has been used"""
+    from exact_amd.model import Cache, DeviceWeights, GraphDecoder, TModel
+    monkeypatch.setattr(ops, "ATT_SHORT_CACHE", 0)
+    monkeypatch.setattr(ops, "ATT_KEYS_WORK", 50 * 128)
+    monkeypatch.setattr(ops, "ATT_EAGER_KEYS", {False: (50, 50), True: (50, 50)})
+    cfg = synth.CONFIGS["tiny-hd128"]
+    tm = TModel(DeviceWeights.synthetic(cfg, 3, DEV), Smax=96)
+    prompt = [(11 * i + 3) % cfg.V for i in range(60)]
+    got, kept = [], []
+    for Smax in (96, 700, 96, 300):
+        cache = Cache(cfg, 1, Smax, tm.dev, cfg.NL)
+        tm.forward(prompt, cache, last_only=True)
+        rows = [[x.clone() for x in tm.decode_rows([5], cache)]]
+        cache.n[0] = 60
+        gd = GraphDecoder(tm, cache, 1)
+        gd.load([5])
+        gd.capture()
+        assert gd._split()
+        rows.append([x.clone() for x in gd.step()])
+        got.append(rows)
+        kept.append((gd, cache))
+    for gd, cache in kept:   # the captured steps still hold their own buffers
+        cache.n[0] = 60
+        gd.load([5])
+        got.append([[x.clone() for x in gd.step()]])
+    assert set(tm.workspace(1).att_work) == {96, 300, 700}
+    assert all(torch.equal(x, y) for rows in got for r in rows for x, y in zip(r, got[0][0]))
