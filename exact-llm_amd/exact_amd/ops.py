@@ -567,7 +567,7 @@ def attention_qkv(t, s, b, cos_t, sin_t, slot, pos, cache, expt, out, H, KV, hd,
     the library may split each head's p.V over obn blocks, one output slice each. keys: the longest row's positions, which a
     caller with short rows in a long cache does well to tell (else half of the cache's): from attention_keys_from() on the call
     is split over the keys (work: its attention_work(), else allocated here), and one launch below. The results are the same
-    either way."""
+    either way. A cache that does not start on 16 bytes, which the split does not take, stays in one launch."""
     R = t.shape[0]
     kq, sk, v = cache
     _need(t, I64, "t", R * (H + 2 * KV) * hd)
@@ -577,7 +577,8 @@ def attention_qkv(t, s, b, cos_t, sin_t, slot, pos, cache, expt, out, H, KV, hd,
     args = (_ptr(t), _ptr(_need(s, I32, "s", R)), _ptr(b), _ptr(cos_t), _ptr(sin_t), _ptr(slot), _ptr(pos), _ptr(kq),
             _ptr(sk), _ptr(v), _ptr(expt), _ptr(out), _ptr(obits))
     Smax = kq.shape[2]
-    if known_keys(keys, Smax) >= attention_keys_from(R, H, KV, hd, Smax) and expt.data_ptr() % 16 == 0:
+    if known_keys(keys, Smax) >= attention_keys_from(R, H, KV, hd, Smax) and not any(
+            a.data_ptr() % 16 for a in (kq, v, expt)):
         work = attention_work(R, H, KV, hd, Smax, t.device) if work is None else work
         _lib.call("exact_attention_decode", *args, obn, _ptr(_need(work, I8, "work")), work.numel(), R, H, KV, hd, Smax, inv,
                   _stream())

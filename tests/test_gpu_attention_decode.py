@@ -198,3 +198,30 @@ def test_cache_longer_than_the_model(monkeypatch):
         got.append([[x.clone() for x in gd.step()]])
     assert set(tm.workspace(1).att_work) == {96, 300, 700}
     assert all(torch.equal(x, y) for rows in got for r in rows for x, y in zip(r, got[0][0]))
+
+
+@pytest.mark.parametrize("H,KV,hd", [(7, 1, 128), (4, 4, 64)])
+def test_caches_off_16_bytes_stay_in_one_launch(H, KV, hd):
+    """keys and values that start 8 bytes past a 16-byte boundary, at positions from which an aligned cache is split"""
+    R, Smax = 2, 1700
+    rng = np.random.default_rng(hd)
+    d = lambda lo, hi, sh, dt: dev(rng.integers(lo, hi, sh), dt)
+    t, s = d(-(1 << 44), 1 << 44, (R, (H + 2 * KV) * hd), I64), d(0, 12, R, I32)
+    kv = (d(-32767, 32768, (R, KV, Smax, hd), I16), d(0, 4, (R, KV, Smax), I32), d(-(1 << 29), 1 << 29, (R, KV, Smax, hd), I64))
+    slot, pos = dev([1, 0], I32), dev([1650, 900], I32)
+    tabs = host_tables(Smax, hd, 1e6)
+    cos, sin, expt = dev(tabs["cos"], I64), dev(tabs["sin"], I64), dev(exp_t(), I32)
+
+    def off(x, n):   # a copy n elements past an aligned address
+        y = torch.empty(x.numel() + n, dtype=x.dtype, device=DEV)[n:].view(x.shape)
+        return y.copy_(x)
+
+    got = []
+    for nk, nv in ((0, 0), (4, 0), (0, 1), (4, 1)):
+        cache = (off(kv[0], nk), kv[1].clone(), off(kv[2], nv))
+        assert (cache[0].data_ptr() % 16, cache[2].data_ptr() % 16) == (2 * nk, 8 * nv)
+        out, ob = torch.full((R, H * hd), -9, dtype=I64, device=DEV), torch.full((R, H, 4), -2, dtype=I32, device=DEV)
+        ops.attention_qkv(t, s, None, cos, sin, slot, pos, cache, expt, out, H, KV, hd, O.inv_sqrt_hd(hd), ob, obn=4, keys=1651)
+        got.append((out, ob.max(-1)[0], *cache))
+    assert 1651 >= ops.attention_keys_from(R, H, KV, hd, Smax)
+    assert all(torch.equal(x, y) for g in got[1:] for x, y in zip(g, got[0]))
