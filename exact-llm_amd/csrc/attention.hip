@@ -147,16 +147,25 @@ __global__ void k_qkv_rope_cache(int64_t* __restrict__ t, const int32_t* __restr
 #ifndef ATT_MR_VPF
 #define ATT_MR_VPF 8
 #endif
+// One block per (row, KV head) for its whole query group (k_attention_gqa): caches longer than ATT_GQA_MIN_S positions, in more
+// (row, head) blocks than the CUs hold at a time of the kernel above, two a CU; groups of 4 heads of 128 in more than one a CU.
+// us a launch, cold caches of 28 layers in turn, positions 100 / 180 / 255 of 256, against a block per (row, head): 280 blocks of
+// 28 heads over 4 (10 rows) 20.3 / 23.4 / 26.8 against 11.8 / 17.0 / 23.0, 504 21.6 / 26.2 / 30.4 against 14.7 / 21.0 / 26.7, 532
+// 21.8 / 26.5 / 30.7 against 21.6 / 31.7 / 41.2; 40 heads over 8, 320 16.4 / 19.4 / 22.0 against 12.9 / 19.5 / 24.9, 520 18.0 /
+// 21.8 / 25.9 against 22.4 / 32.3 / 41.9; 32 heads over 8, 288 15.0 / 18.3 / 21.4 against 15.4 / 22.1 / 28.3; heads of 64, 14 over
+// 2, 280 19.0 / 20.7 / 22.4 against 9.0 / 10.3 / 11.6. (From 193 positions of hd 128 exact_attention_decode is faster than both:
+// 19.3, 20 and 19.6 at 255 in the first, fourth and sixth of these.)
 #ifndef ATT_GQA
 #define ATT_GQA 1
 #endif
 #ifndef ATT_GQA_NT
 #define ATT_GQA_NT 512
 #endif
-// ... for caches longer than this (14B bs8, cold caches of 48 layers in turn: at 256 positions 23.2 against 25.1 us
-// a launch, at 148 positions 18.8 against 17.1, decode 5.37 against 5.28 ms a step; 1024-thread blocks: slower still)
 #ifndef ATT_GQA_MIN_S
 #define ATT_GQA_MIN_S 192
+#endif
+#ifndef ATT_GQA_BLOCKS
+#define ATT_GQA_BLOCKS 512
 #endif
 #ifndef ATT_MR_GT
 #define ATT_MR_GT 1
@@ -987,8 +996,8 @@ extern "C" int exact_attention_qkv_split(const int64_t* t, const int32_t* s, con
   // ... and, for query groups of 4, 5, 7 or 8 heads over caches of at most 256 positions, one block per (row, KV
   // head, dimension slice) for the whole group
   const int grp = H / KV;
-  const bool gqa = ATT_GQA && blocks > ATT_WIDE_BLOCKS && hd % 64 == 0 && hd <= 128 && Smax > ATT_GQA_MIN_S && Smax <= 256 &&
-                   (grp == 4 || grp == 5 || grp == 7 || grp == 8);
+  const bool gqa = ATT_GQA && blocks > (grp == 4 && hd == 128 ? ATT_WIDE_BLOCKS : ATT_GQA_BLOCKS) && hd % 64 == 0 && hd <= 128 &&
+                   Smax > ATT_GQA_MIN_S && Smax <= 256 && (grp == 4 || grp == 5 || grp == 7 || grp == 8);
   if (gqa) {
     const int gds = att_qkv_ds(obn, (int64_t)R * KV, hd);
     if (grp == 4) att_gqa_go<4>(gds, ATT_QKV_ARGS);

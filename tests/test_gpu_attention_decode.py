@@ -225,3 +225,30 @@ def test_caches_off_16_bytes_stay_in_one_launch(H, KV, hd):
         got.append((out, ob.max(-1)[0], *cache))
     assert 1651 >= ops.attention_keys_from(R, H, KV, hd, Smax)
     assert all(torch.equal(x, y) for g in got[1:] for x, y in zip(g, got[0]))
+
+
+@pytest.mark.parametrize("H,KV,hd", [(4, 1, 128), (5, 1, 128), (14, 2, 128), (8, 1, 128), (8, 2, 64), (7, 1, 64)])
+@pytest.mark.parametrize("blocks", [257, 512, 513])
+@pytest.mark.parametrize("Smax,obn", [(193, 4), (256, 1)])
+def test_batch_attention_around_the_grouped_kernels_line(H, KV, hd, blocks, Smax, obn):
+    """Rows in one more (row, head) block than the CUs hold, and in as many as, and more than, from which a block takes a whole
+    group: equal to the two launches"""
+    R = -(-blocks // H) if blocks != 512 else 512 // H
+    rng = np.random.default_rng(R + hd)
+    d = lambda lo, hi, sh, dt: dev(rng.integers(lo, hi, sh), dt)
+    t, s = d(-(1 << 44), 1 << 44, (R, (H + 2 * KV) * hd), I64), d(0, 12, R, I32)
+    c_a = (d(-32767, 32768, (R, KV, Smax, hd), I16), d(0, 4, (R, KV, Smax), I32), d(-(1 << 29), 1 << 29, (R, KV, Smax, hd), I64))
+    c_b = tuple(x.clone() for x in c_a)
+    slot, pos = dev(rng.permutation(R), I32), d(0, Smax, R, I32)
+    pos[0], pos[1] = 0, Smax - 1
+    tabs = host_tables(Smax, hd, 1e6)
+    cos, sin, expt = dev(tabs["cos"], I64), dev(tabs["sin"], I64), dev(exp_t(), I32)
+    qq, sq = torch.empty((R, H * hd), dtype=I16, device=DEV), torch.empty((R, H), dtype=I32, device=DEV)
+    out_a, out_b = (torch.full((R, H * hd), x, dtype=I64, device=DEV) for x in (-7, -9))
+    ob_a, ob_b = torch.full((R, H), -1, dtype=I32, device=DEV), torch.full((R, H, obn), -2, dtype=I32, device=DEV)
+    inv = O.inv_sqrt_hd(hd)
+    ops.qkv_rope_cache(t, s, None, cos, sin, slot, pos, c_a, qq, sq, H, KV, hd)
+    ops.attention(qq, sq, c_a, slot, pos, expt, out_a, H, KV, hd, inv, ob_a)
+    ops.attention_qkv(t, s, None, cos, sin, slot, pos, c_b, expt, out_b, H, KV, hd, inv, ob_b, obn=obn, keys=1)
+    assert torch.equal(out_a, out_b) and torch.equal(ob_b.max(-1)[0], ob_a)
+    assert all(torch.equal(x, y) for x, y in zip(c_a, c_b))
