@@ -641,23 +641,31 @@ def temp_num(temp):
     return int(round((1 << 16) / temp))
 
 
-# From this many logits a row is split over blocks (four launches); below, one block a row walks it (one launch). us a call at
-# 4096 / 6000 / 8192 / 16384 / 151936 logits, one row: 13.5 / 17.7 / 21.8 / 38.3 / 310 in one launch; 19.1 / 18.9 / 19.1 /
-# 19.1 / 17.9 split (bound by the host's four launches; 14.7 / 15.0 / 15.0 / 15.2 / 15.7 in a graph). Eight rows of 151936:
-# 311 and 20.6.
-SAMPLE_SPLIT_FROM = 6144
+# From this many logits a row is split over blocks (four launches, bound by the host: 20 to 24 us a call), below and in calls of
+# more rows one block a row walks it (one launch). us a call, one launch and split: one row of 6144 / 8000 / 16384 / 151936 logits
+# 18.8 / 22.4 / 38.6 / 305 and 22.0 / 20.5 / 20.0 / 20.4 (in a graph 18.2 / 18.6 / 18.6 / 19.1); 256 rows of 10240 / 16384 / 49152
+# 28.8 / 49.3 / 149 and 31.7 / 41.8 / 95.5; 1024 rows of 16384 / 151936 143 / 1536 and 123 / 1288. A split call's workspace is
+# half as large as its logits, so that calls of many rows take it in groups of rows.
+SAMPLE_SPLIT_FROM = 7168
+SAMPLE_SPLIT_MANY, SAMPLE_SPLIT_FROM_MANY = 128, 16384   # rows above which a row is split from as many logits
+SAMPLE_WORK_BYTES = 256 << 20
 
 
 def sample(lg, seed, step, tnum, expt, ids, p_out=None):
     """ids[r] = sample_int(lg[r], seed, step[r], tnum) (exact_llm.py:256-259), on the device."""
     R, V = lg.shape
-    args = (_ptr(_need(lg, I64, "lg")), R, V, ctypes.c_uint64(seed), _ptr(_need(step, I32, "step", R)), tnum, _ptr(expt),
-            _ptr(_need(ids, I32, "ids", R)), _ptr(p_out))
-    if V >= SAMPLE_SPLIT_FROM:
-        work = torch.empty(_lib.load().exact_sample_workspace(R, V), dtype=I8, device=lg.device)
-        _lib.call("exact_sample_split", *args, _ptr(work), work.numel(), _stream())
-    else:
-        _lib.call("exact_sample", *args, _stream())
+    seed = ctypes.c_uint64(seed)
+    _need(lg, I64, "lg"), _need(step, I32, "step", R), _need(ids, I32, "ids", R)
+    if V < SAMPLE_SPLIT_FROM or (R > SAMPLE_SPLIT_MANY and V < SAMPLE_SPLIT_FROM_MANY):
+        _lib.call("exact_sample", _ptr(lg), R, V, seed, _ptr(step), tnum, _ptr(expt), _ptr(ids), _ptr(p_out), _stream())
+        return ids
+    row = _lib.load().exact_sample_workspace(1, V)   # the workspace of n rows is n of these
+    n = min(R, max(1, SAMPLE_WORK_BYTES // row))
+    work = torch.empty(n * row, dtype=I8, device=lg.device)
+    for r in range(0, R, n):
+        at = lambda t, size: None if t is None else ctypes.c_void_p(t.data_ptr() + r * size)
+        _lib.call("exact_sample_split", at(lg, 8 * V), min(n, R - r), V, seed, at(step, 4), tnum, _ptr(expt), at(ids, 4),
+                  at(p_out, 8 * V), _ptr(work), work.numel(), _stream())
     return ids
 
 

@@ -141,3 +141,38 @@ def test_split_rows_of_no_exponential_match_the_one_block_kernel(table):
         finally:
             ops.SAMPLE_SPLIT_FROM = old
         assert (host(ids) == V).all() and not host(pd).any(), lim
+
+
+@pytest.mark.parametrize("R,rows", [(7, 3), (6, 2), (5, 1), (4, 9)])
+@pytest.mark.parametrize("with_p", [False, True])
+def test_split_rows_in_groups_match_one_block_a_row(R, rows, with_p, monkeypatch):
+    """calls whose workspace is bounded to so many rows (a last group of fewer among them), ids over the steps' own array"""
+    V, seed, tnum = 9000, 21, ops.temp_num(0.8)
+    rng = np.random.default_rng(R)
+    lg = torch.tensor(rng.integers(-(4 << 16), 4 << 16, (R, V)), device=DEV)
+    expt = torch.tensor(exp_t(), dtype=I32, device=DEV)
+    monkeypatch.setattr(ops, "SAMPLE_WORK_BYTES", _lib.load().exact_sample_workspace(rows, V) + 5)
+    got = []
+    for lim in (V + 1, V):
+        monkeypatch.setattr(ops, "SAMPLE_SPLIT_FROM", lim)
+        ids = torch.arange(R, dtype=I32, device=DEV) * 3 + 1
+        pd = torch.full((R, V), -1, dtype=I64, device=DEV) if with_p else None
+        torch.cuda.synchronize()
+        ops.sample(lg, seed, ids, tnum, expt, ids, pd)
+        got.append((host(ids), host(pd) if with_p else None))
+    assert np.array_equal(got[0][0], got[1][0]) and (not with_p or np.array_equal(got[0][1], got[1][1]))
+
+
+def test_many_split_rows_keep_the_workspace_bounded():
+    """the memory that a call takes beside its logits"""
+    R, V = 600, 152064
+    lg = torch.zeros((R, V), dtype=I64, device=DEV)
+    step, ids = torch.arange(R, dtype=I32, device=DEV), torch.zeros(R, dtype=I32, device=DEV)
+    expt = torch.tensor(exp_t(), dtype=I32, device=DEV)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    ops.sample(lg, 3, step, ops.temp_num(1.0), expt, ids)
+    assert torch.cuda.max_memory_allocated() - before <= ops.SAMPLE_WORK_BYTES + (2 << 20)
+    got = host(ids)
+    assert ((0 <= got) & (got < V)).all() and len(set(got.tolist())) > R // 2   # equal logits: tokens over the whole row
