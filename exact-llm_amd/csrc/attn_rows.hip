@@ -146,7 +146,7 @@ extern "C" int exact_attention_rows(const int16_t* qq, const int32_t* sq, const 
                                     void* stream) {
   if (!qq || !sq || !kq || !sk || !v || !slot || !pos || !exp_t || !out) return EXACT_E_ARG;
   if (R <= 0 || H <= 0 || KV <= 0 || H % KV || hd <= 0 || Smax <= 0 || nkeys <= 0) return EXACT_E_ARG;
-  if ((hd != 64 && hd != 128) || nkeys > 128 || (int64_t)R * H > INT32_MAX / 2) return EXACT_E_UNSUPPORTED;
+  if ((hd != 64 && hd != 128) || nkeys > 128 || Smax > 8192 || (int64_t)R * H > INT32_MAX / 2) return EXACT_E_UNSUPPORTED;
   if (((uintptr_t)qq | (uintptr_t)kq | (uintptr_t)v | (uintptr_t)out) & 15) return EXACT_E_UNSUPPORTED;
   const dim3 grid((uint32_t)cdiv((int64_t)R * H, ROWS_WAVES)), block(ROWS_WAVES * 64);
 #define ROWS_GO(HD, NK)                                                                                                  \

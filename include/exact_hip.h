@@ -294,8 +294,8 @@ int exact_attention(const int16_t* qq, const int32_t* sq, const int16_t* kq, con
                     int64_t* out, int32_t* obits, int32_t R, int32_t H, int32_t KV, int32_t hd, int32_t Smax,
                     int32_t INV, void* stream);
 
-/* exact_attention for rows whose positions are all below nkeys <= 128, hd 64 or 128, qq, kq, v and out 16-byte aligned
- * (otherwise EXACT_E_UNSUPPORTED): a wave per (row, head). Same results. */
+/* exact_attention for rows whose positions are all below nkeys <= 128, hd 64 or 128, Smax <= 8192 (as exact_attention), qq, kq,
+ * v and out 16-byte aligned (otherwise EXACT_E_UNSUPPORTED): a wave per (row, head). Same results. */
 int exact_attention_rows(const int16_t* qq, const int32_t* sq, const int16_t* kq, const int32_t* sk,
                          const int64_t* v, const int32_t* slot, const int32_t* pos, const int32_t* exp_t,
                          int64_t* out, int32_t* obits, int32_t R, int32_t H, int32_t KV, int32_t hd, int32_t Smax,

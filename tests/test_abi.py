@@ -66,3 +66,14 @@ def test_host_side_validation_rejects_bad_shapes_without_launching():
     assert lib.exact_gemv(None, fake, fake, fake, 64, 128, None) == 1                            # exact::gemv: null x
     assert lib.exact_gemv(fake, fake, fake, fake, 64, 200, None) == 2                            # K % 128
     assert lib.exact_gemv(fake + 8, fake, fake, fake, 64, 128, None) == 2                        # x not 16-byte aligned
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
+@pytest.mark.parametrize("hd", [64, 128])
+def test_short_prompts_in_too_long_caches_are_refused_on_every_path(hd):
+    """caches past exact_attention's limit, however few of their positions a call asks for"""
+    lib, fake = _lib.load(), 1 << 20
+    head = (fake,) * 9 + (None, 4, 4, 2, hd)
+    assert lib.exact_attention(*head, 8193, 8192, None) == 2
+    assert lib.exact_attention_rows(*head, 8193, 10, 8192, None) == 2
+    assert lib.exact_attention_decode_workspace(4, 4, 2, hd, 8193) == 0
