@@ -660,9 +660,9 @@ def sample(lg, seed, step, tnum, expt, ids, p_out=None):
         _lib.call("exact_sample", _ptr(lg), R, V, seed, _ptr(step), tnum, _ptr(expt), _ptr(ids), _ptr(p_out), _stream())
         return ids
     row = _lib.load().exact_sample_workspace(1, V)   # the workspace of n rows is n of these
-    n = min(R, max(1, SAMPLE_WORK_BYTES // row))
+    n = max(1, min(R, SAMPLE_WORK_BYTES // row))
     work = torch.empty(n * row, dtype=I8, device=lg.device)
-    for r in range(0, R, n):
+    for r in range(0, max(R, 1), n):   # no rows: refused by the call
         at = lambda t, size: None if t is None else ctypes.c_void_p(t.data_ptr() + r * size)
         _lib.call("exact_sample_split", at(lg, 8 * V), min(n, R - r), V, seed, at(step, 4), tnum, _ptr(expt), at(ids, 4),
                   at(p_out, 8 * V), _ptr(work), work.numel(), _stream())

@@ -176,3 +176,10 @@ def test_many_split_rows_keep_the_workspace_bounded():
     assert torch.cuda.max_memory_allocated() - before <= ops.SAMPLE_WORK_BYTES + (2 << 20)
     got = host(ids)
     assert ((0 <= got) & (got < V)).all() and len(set(got.tolist())) > R // 2   # equal logits: tokens over the whole row
+
+
+@pytest.mark.parametrize("V", [100, 9000, 20000])
+def test_no_rows_are_refused(V):
+    z = lambda *sh, dt=I32: torch.zeros(sh, dtype=dt, device=DEV)
+    with pytest.raises(ops.ExactError, match="bad argument"):
+        ops.sample(z(0, V, dt=I64), 1, z(0), ops.temp_num(1.0), torch.tensor(exp_t(), dtype=I32, device=DEV), z(0))
