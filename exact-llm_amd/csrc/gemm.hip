@@ -727,6 +727,15 @@ __global__ __launch_bounds__(256) void k_split_rows_a16(const int16_t* __restric
 }
 
 // gathered int8 rows: x8[p] = x[row_map[p]] (16 bytes per thread; K % 16 == 0)
+__global__ __launch_bounds__(256) void k_gather_rows_a8(const int8_t* __restrict__ x, int8_t* __restrict__ x8, int64_t P, int K,
+                                                        const int32_t* __restrict__ row_map) {
+  const int64_t n16 = P * (K / 16);
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n16; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t p = i / (K / 16), c = (i - p * (K / 16)) * 16;
+    *reinterpret_cast<v4i*>(x8 + p * K + c) = *reinterpret_cast<const v4i*>(x + (int64_t)row_map[p] * K + c);
+  }
+}
+
 // Tile of the A8 kernel by its A rows M (digit rows of int16): up to 64 rows (prompts of 17 to 32 tokens) 64 x 64, one wave, three
 // blocks a CU; up to 128 rows 128 x 128, two blocks a CU; 256 x 128 beyond. 37888 x 3584 at 32 tokens: 31.4 us in 64 x 64, 40.0
 // in 64 x 128, 40.3 in 128 x 128, whose waves of padding rows compute as well; at 41 tokens 60.0, 56.6 and 40.3.
@@ -964,7 +973,7 @@ extern "C" int exact_gemm_g128_experts(const void* x, int32_t abits, const int32
                                        const int32_t* chunk_e, const int32_t* chunk_p0, const int32_t* chunk_n,
                                        const int32_t* nchunks, int32_t max_chunks, int64_t* t, int32_t P, int32_t N, int32_t K,
                                        void* stream) {
-  if (!x || !wp || !mp || !x8 || !chunk_e || !chunk_p0 || !chunk_n || !nchunks || !t) return EXACT_E_ARG;
+  if (!x || !wp || !mp || (abits == 15 && !x8) || !chunk_e || !chunk_p0 || !chunk_n || !nchunks || !t) return EXACT_E_ARG;
   if (P <= 0 || N <= 0 || K <= 0 || max_chunks <= 0 || w_stride <= 0 || m_stride <= 0) return EXACT_E_ARG;
   if (abits == 15 && !colterm) return EXACT_E_ARG;
   if ((abits != 15 && abits != 7) || K % 128 || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(x8) & 15) ||
@@ -973,15 +982,21 @@ extern "C" int exact_gemm_g128_experts(const void* x, int32_t abits, const int32
   const int64_t rows = (abits == 15 ? 2 : 1) * (int64_t)P;
   if (rows * K >= (1LL << 32)) return EXACT_E_UNSUPPORTED;   // 32-bit buffer offsets
   hipStream_t st = as_stream(stream);
+  const int blocks = (int)std::min<int64_t>(((int64_t)P * (K / 16) + 255) / 256, 8192);
   if (abits == 15) {
-    const int blocks = (int)std::min<int64_t>(((int64_t)P * (K / 16) + 255) / 256, 8192);
     hipLaunchKernelGGL(k_split_rows_a16, dim3(blocks), dim3(256), 0, st, static_cast<const int16_t*>(x), x8, (int64_t)P, K,
                        row_map);
     return gemm_launch_experts<GEMM_A8P_CFG, true>(x8, nullptr, wp, mp, w_stride, m_stride, colterm, chunk_e, chunk_p0, chunk_n,
                                                    nchunks, max_chunks, t, (int)rows, N, K, st);
   }
-  return gemm_launch_experts<GEMM_A8P_CFG, false>(static_cast<const int8_t*>(x), row_map, wp, mp, w_stride, m_stride, nullptr,
-                                                  chunk_e, chunk_p0, chunk_n, nchunks, max_chunks, t, (int)rows, N, K, st);
+  const int8_t* xa = static_cast<const int8_t*>(x);
+  if (row_map && x8) {   // x may have any number of rows: the GEMM's 32-bit offsets reach P of them
+    hipLaunchKernelGGL(k_gather_rows_a8, dim3(blocks), dim3(256), 0, st, xa, x8, (int64_t)P, K, row_map);
+    xa = x8;
+    row_map = nullptr;
+  }
+  return gemm_launch_experts<GEMM_A8P_CFG, false>(xa, row_map, wp, mp, w_stride, m_stride, nullptr, chunk_e, chunk_p0, chunk_n,
+                                                  nchunks, max_chunks, t, (int)rows, N, K, st);
 }
 
 extern "C" int exact_gemm_g128_experts_digits(const int8_t* x8, const int32_t* row_map, const int8_t* wp, const int16_t* mp,

@@ -873,11 +873,13 @@ def gemm_experts(x, abits, row_map, lin, disp, out, P):
     _need(out, I64, "out", P * lin.N)
     if x.shape[1] != lin.K or out.shape[1] != lin.N:
         raise ExactError(f"gemm_experts: x {tuple(x.shape)}, out {tuple(out.shape)} against ({lin.N}, {lin.K})")
-    need = (2 if abits == 15 else 1) * P * lin.K
-    ws = _EXPERT_ROWS.get(x.device)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(need, dtype=I8, device=x.device)
-        _EXPERT_ROWS[x.device] = ws
+    ws = None
+    if abits == 15 or (row_map is not None and x.numel() >= 1 << 32):   # digit rows; int8 rows past the GEMM's 32-bit offsets
+        need = (2 if abits == 15 else 1) * P * lin.K
+        ws = _EXPERT_ROWS.get(x.device)
+        if ws is None or ws.numel() < need:
+            ws = torch.empty(need, dtype=I8, device=x.device)
+            _EXPERT_ROWS[x.device] = ws
     ct = expert_colterm(lin) if abits == 15 else None
     _lib.call("exact_gemm_g128_experts", _ptr(x), abits, _ptr(row_map), _ptr(lin.wp), _ptr(lin.mp), lin.w_stride, lin.m_stride,
               _ptr(ct), _ptr(ws), _ptr(disp["chunk_e"]), _ptr(disp["chunk_p0"]), _ptr(disp["chunk_n"]), _ptr(disp["nchunks"]),

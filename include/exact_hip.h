@@ -176,7 +176,8 @@ int exact_gemv_g128_norm_swiglu(const int64_t* x_in, int64_t* x_out, const int64
  * dispatched pairs, t[p] = x[row_map[p]] . W_e with e = chunk_e[c] (row_map NULL: x row p), expert e's packed
  * linear at wp + e * w_stride, mp + e * m_stride. int16 x runs as interleaved digit rows (as
  * exact_gemm_g128_a16) and needs colterm (NE, N) = each expert's sum_g colsum_g M_g. x8: workspace of 2 P K
- * (int16) or P K (int8; not used) bytes. max_chunks: the length of the chunk arrays (launch size).
+ * (int16) or P K (int8) bytes; with int8 it may be NULL if x takes fewer than 2^32 bytes: the GEMM then reads
+ * row row_map[p] itself, with no launch that gathers the rows. max_chunks: the length of the chunk arrays (launch size).
  * Replaces the per-expert loop of MoEInt.moe (moe_exact_kaggle.py:460-464) for prefill-sized pair counts. */
 int exact_gemm_g128_experts(const void* x, int32_t abits, const int32_t* row_map, const int8_t* wp, const int16_t* mp,
                             int64_t w_stride, int64_t m_stride, const int64_t* colterm, int8_t* x8, const int32_t* chunk_e,

@@ -455,3 +455,21 @@ def test_expert_gemm_of_digit_rows_matches_int16_rows(R, NE, k, N, K):
     ops.gemm_experts(split(x), 15, d["pair_row"], lin, d, got, P)
     ops.gemm_experts(split(x[host(d["pair_row"])]), 15, None, lin, d, ordered, P)
     assert torch.equal(want, got) and torch.equal(want, ordered)
+
+
+def test_expert_gemm_of_int8_rows_beyond_4_gib():
+    """row_map reaches rows whose offsets need more than 32 bits; smaller activations take no workspace"""
+    R, NE, k, N, K = 24, 4, 2, 64, 128
+    rng = np.random.default_rng(5)
+    lin, e_sel, _, _, x = _expert_case(rng, 7, R, NE, k, N, K, list(range(NE)))
+    P, xd = R * k, dev(x, torch.int8)
+    d = _dispatch(e_sel, NE, k, ops.EXPERT_CHUNK[7], 7)
+    want, got = (torch.full((P, N), f, dtype=I64, device=DEV) for f in (-1, -2))
+    ops._EXPERT_ROWS.clear()
+    ops.gemm_experts(xd, 7, d["pair_row"], lin, d, want, P)
+    assert not ops._EXPERT_ROWS
+    rows = (1 << 32) // K + 7
+    big = torch.zeros((rows, K), dtype=torch.int8, device=DEV)
+    big[rows - R:] = xd
+    ops.gemm_experts(big, 7, d["pair_row"] + (rows - R), lin, d, got, P)
+    assert torch.equal(want, got)
