@@ -700,7 +700,8 @@ class TModel:
                     cg = torch.cuda.CUDAGraph()
                     with torch.cuda.graph(cg):
                         self.forward_rows(ws, last_only=last_only, keys=p0 + T)
-                    self._graphs[key] = (cg, cache)   # the graph holds the cache's buffers
+                    # the graph holds the cache's buffers, and the attention workspace that a longer prompt may replace
+                    self._graphs[key] = (cg, cache, self._pws)
                     while len(self._graphs) > self.PREFILL_GRAPHS:
                         self._graphs.popitem(last=False)
         finally:

@@ -254,3 +254,21 @@ def test_prompts_over_stale_totals(name, abits, T):
         assert all(torch.equal(u, v) for x, y in zip(c0.layers, c1.layers) for u, v in zip(x, y))
         la, lb = tm.decode_rows([3], c0)[0], fresh.decode_rows([3], c1)[0]
         assert torch.equal(la, lb)
+
+
+def test_captured_prompts_keep_their_attention_workspace():
+    """A longer prompt replaces the model's prefill-attention workspace; a captured shorter one still owns the one that its
+    kernels write, so that neither its result nor memory allocated since changes"""
+    cfg = synth.CONFIGS["tiny"]
+    tm = TModel(DeviceWeights.synthetic(cfg, 21, "cuda"), Smax=700)
+    cache, ids = tm.new_cache(B=1), helpers.prompt(1, 200, cfg.V)
+    want = host(tm.forward(ids, cache, graph=True))
+    old = tm._pws[1]
+    size, addr = old.numel(), old.data_ptr()
+    del old
+    tm.forward(helpers.prompt(2, 600, cfg.V), tm.new_cache(B=1))
+    assert tm._pws[1].data_ptr() != addr
+    others = [torch.full((size,), 77, dtype=torch.int8, device="cuda") for _ in range(4)]
+    cache.n[0] = 0
+    assert np.array_equal(host(tm.forward(ids, cache, graph=True)), want)
+    assert all((o == 77).all() for o in others)
