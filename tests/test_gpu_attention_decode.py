@@ -72,19 +72,32 @@ def test_split_extreme_values_and_tables():
     assert not compare(4, 2, 128, 200, [199], 6, table=np.zeros_like(exp_t())).any()
 
 
-def test_split_positions_outside_the_cache_give_zeros():
-    H, KV, hd, Smax = 4, 2, 64, 256
-    z = lambda *sh, dt=I64: torch.zeros(sh, dtype=dt, device=DEV)
-    cache = (z(2, KV, Smax, hd, dt=I16), z(2, KV, Smax, dt=I32), z(2, KV, Smax, hd))
-    out, ob = torch.full((2, H * hd), -1, dtype=I64, device=DEV), torch.full((2, H, 4), -1, dtype=I32, device=DEV)
-    t = torch.full((2, (H + 2 * KV) * hd), 1 << 40, dtype=I64, device=DEV)
-    ops.attention_qkv(t, z(2, dt=I32), None, z(Smax, hd), z(Smax, hd), dev([0, 1], I32), dev([-1, Smax], I32), cache,
-                      dev(exp_t(), I32), out, H, KV, hd, O.inv_sqrt_hd(hd), ob, obn=4, keys=Smax,
-                      work=ops.attention_work(2, H, KV, hd, Smax, DEV))
-    ops._lib.call("exact_attention_decode", *(ops._ptr(x) for x in (t, z(2, dt=I32), None, z(Smax, hd), z(Smax, hd),
-                  dev([0, 1], I32), dev([-1, Smax], I32), *cache, dev(exp_t(), I32), out, ob)), 4,
-                  ops._ptr(ops.attention_work(2, H, KV, hd, Smax, DEV)), 1 << 30, 2, H, KV, hd, Smax, 1, ops._stream())
-    assert not out.any() and not ob.any() and not any(x.any() for x in cache)
+@pytest.mark.parametrize("hd,obn", [(64, 4), (128, 1)])
+def test_split_positions_outside_the_cache_give_zeros(hd, obn):
+    """rows at positions -1 and Smax, on either path: outputs and bit lengths 0, the cache as it was"""
+    H, KV, Smax = 4, 2, 256
+    rng = np.random.default_rng(hd)
+    d = lambda lo, hi, sh, dt: dev(rng.integers(lo, hi, sh), dt)
+    kv = (d(-32767, 32768, (2, KV, Smax, hd), I16), d(0, 4, (2, KV, Smax), I32), d(-(1 << 29), 1 << 29, (2, KV, Smax, hd), I64))
+    t, s = d(-(1 << 44), 1 << 44, (2, (H + 2 * KV) * hd), I64), d(0, 12, 2, I32)
+    tabs = host_tables(Smax, hd, 1e6)
+    cos, sin, expt = dev(tabs["cos"], I64), dev(tabs["sin"], I64), dev(exp_t(), I32)
+    slot, pos, inv = dev([0, 1], I32), dev([-1, Smax], I32), O.inv_sqrt_hd(hd)
+    work = ops.attention_work(2, H, KV, hd, Smax, DEV).fill_(0x5A)
+
+    def one_launch(cache, out, ob):
+        ops.attention_qkv(t, s, None, cos, sin, slot, pos, cache, expt, out, H, KV, hd, inv, ob, obn=obn, keys=1)
+
+    def split(cache, out, ob):
+        ops._lib.call("exact_attention_decode", *(ops._ptr(x) for x in (t, s, None, cos, sin, slot, pos, *cache, expt, out, ob)),
+                      obn, ops._ptr(work), work.numel(), 2, H, KV, hd, Smax, inv, ops._stream())
+
+    for path in (one_launch, split):
+        cache = tuple(x.clone() for x in kv)
+        out, ob = torch.full((2, H * hd), -1, dtype=I64, device=DEV), torch.full((2, H, obn), -1, dtype=I32, device=DEV)
+        path(cache, out, ob)
+        assert not out.any() and not ob.any(), path.__name__
+        assert all(torch.equal(x, y) for x, y in zip(cache, kv)), path.__name__
 
 
 @pytest.mark.parametrize("B", [1, 3])

@@ -661,3 +661,28 @@ def test_swiglu_in_the_prefill_gemm_matches_its_separate_launches(thr, R, I, K):
         assert np.array_equal(host(xa)[i], q[0]) and int(host(sa)[i]) == int(np.ravel(e)[0]), i
     pn = host(part)
     assert (pn <= 31).any() and (pn > 31).any()
+
+
+@pytest.mark.parametrize("abits,R", [(15, 17), (15, 31), (15, 32), (15, 33), (7, 17), (7, 63), (7, 64), (7, 65)])
+@pytest.mark.parametrize("N,K", [(61, 128), (130, 896), (500, 2048), (1152, 1664)])
+def test_wide_group_scales_in_the_64_row_tiles(abits, R, N, K):
+    """Two scale planes in the GEMM's 64 x 64 tiles (up to 64 A rows, two for an int16 row) and one row past them: one K group
+    and several, whole and ragged columns; every entry, into cleared totals and, where it does not add, into stale ones"""
+    r = np.random.default_rng(R * N + K)
+    w = r.integers(-127, 128, (K, N)).astype(np.int8)
+    M = r.integers(0, 1 << 21, (K // 128, N))
+    M[0, :3] = [0, (1 << 15) - 1, 1 << 15]
+    lin = ops.pack_group_linear(w, M, DEV)
+    assert lin.mh is not None
+    lim = (1 << abits) - 1
+    xq = r.integers(-lim, lim + 1, (R, K))
+    xq[0, :2] = [lim, -lim]
+    want, x = oracle_t(xq, w, M), dev(xq, I16 if abits == 15 else I8)
+    x8 = dev(np.stack([xq >> 8, (xq & 255) - 128], 1).reshape(2 * R, K), I8) if abits == 15 else None
+    assert np.array_equal(host(ops.linear_t(x, abits, lin, torch.full((R, N), 7, dtype=I64, device=DEV))), want)
+    for digits in {None, x8}:
+        t = torch.zeros((R, N), dtype=I64, device=DEV)
+        assert np.array_equal(host(ops.linear_t(x, abits, lin, t, zeroed=True, x8=digits)), want)
+    if not ops.linear_adds(R, abits, lin):
+        t = torch.full((R, N), 7, dtype=I64, device=DEV)
+        assert np.array_equal(host(ops.linear_t(x, abits, lin, t, zeroed=True, x8=x8)), want)
