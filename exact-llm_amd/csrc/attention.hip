@@ -7,7 +7,6 @@
 #include "exact_common.h"
 #include "abi_util.h"
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef short s2v __attribute__((ext_vector_type(2)));
 
 // a.lo b.lo + a.hi b.hi of two int16 pairs (v_dot2_i32_i16): exact in int32 for |a|, |b| <= 32767

@@ -16,8 +16,6 @@
 #include "exact_common.h"
 #include "abi_util.h"
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-
 namespace exact {
 
 #define DEC_CK 128        // keys a block: 16 a wave in k_dec_scores, 32 in k_dec_pv
@@ -25,18 +23,6 @@ namespace exact {
 #define DEC_C_THREADS 256
 #define DEC_SMAX 8192
 #define DEC_NCH (DEC_SMAX / DEC_CK)   // chunks of the longest cache: one a lane
-
-// int16 -> (hi, lo - 128) int8 digits of 16 values held in two 16-byte chunks
-__device__ __forceinline__ void dec_digits(v4i p0, v4i p1, v4i& hi, v4i& lo) {
-  hi[0] = __builtin_amdgcn_perm(p0[1], p0[0], 0x07050301u);
-  hi[1] = __builtin_amdgcn_perm(p0[3], p0[2], 0x07050301u);
-  hi[2] = __builtin_amdgcn_perm(p1[1], p1[0], 0x07050301u);
-  hi[3] = __builtin_amdgcn_perm(p1[3], p1[2], 0x07050301u);
-  lo[0] = __builtin_amdgcn_perm(p0[1], p0[0], 0x06040200u) ^ 0x80808080;
-  lo[1] = __builtin_amdgcn_perm(p0[3], p0[2], 0x06040200u) ^ 0x80808080;
-  lo[2] = __builtin_amdgcn_perm(p1[1], p1[0], 0x06040200u) ^ 0x80808080;
-  lo[3] = __builtin_amdgcn_perm(p1[3], p1[2], 0x06040200u) ^ 0x80808080;
-}
 
 // grid (ceil(Smax / DEC_CK), KV, R). sc[(r H + h) Sp + key]: the scores of the keys 0 .. pos[r]. Blocks of chunks past the
 // position leave at once. q.k on the matrix cores from int8 digits x = 256 hi + lo + 128 (every digit sum is below 2^22):
@@ -151,7 +137,7 @@ __global__ __launch_bounds__(DEC_A_THREADS) void k_dec_scores(
 #pragma unroll
   for (int i = 0; i < KS; ++i) {
     v4i khi, klo;
-    dec_digits(kk[i][0], kk[i][1], khi, klo);
+    split_digits(kk[i][0], kk[i][1], khi, klo);
     const v4i q = *reinterpret_cast<const v4i*>(&qd[col >> 3][hb][64 * i + 16 * qt]);
     ch = __builtin_amdgcn_mfma_i32_16x16x64_i8(khi, q, ch, 0, 0, 0);
     cl = __builtin_amdgcn_mfma_i32_16x16x64_i8(klo, q, cl, 0, 0, 0);

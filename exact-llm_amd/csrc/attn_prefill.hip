@@ -20,25 +20,11 @@
 #include "exact_common.h"
 #include "abi_util.h"
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 namespace exact {
 
-
 #define AP_TN 4608   // exp entries in LDS; the fast path needs the table to be zero from entry AP_TN - 2 on
-
-// int16 -> (hi, lo - 128) int8 digits of 16 values held in two 16-byte chunks
-__device__ __forceinline__ void split_digits(v4i p0, v4i p1, v4i& hi, v4i& lo) {
-  hi[0] = __builtin_amdgcn_perm(p0[1], p0[0], 0x07050301u);
-  hi[1] = __builtin_amdgcn_perm(p0[3], p0[2], 0x07050301u);
-  hi[2] = __builtin_amdgcn_perm(p1[1], p1[0], 0x07050301u);
-  hi[3] = __builtin_amdgcn_perm(p1[3], p1[2], 0x07050301u);
-  lo[0] = __builtin_amdgcn_perm(p0[1], p0[0], 0x06040200u) ^ 0x80808080;
-  lo[1] = __builtin_amdgcn_perm(p0[3], p0[2], 0x06040200u) ^ 0x80808080;
-  lo[2] = __builtin_amdgcn_perm(p1[1], p1[0], 0x06040200u) ^ 0x80808080;
-  lo[3] = __builtin_amdgcn_perm(p1[3], p1[2], 0x06040200u) ^ 0x80808080;
-}
 
 // sum of the 16 int16 values in two 16-byte chunks
 __device__ __forceinline__ int sum16(v4i p0, v4i p1) {

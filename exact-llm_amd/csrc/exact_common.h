@@ -22,6 +22,8 @@
 #define EXACT_TILE_GN 1
 #endif
 
+typedef int v4i __attribute__((ext_vector_type(4)));
+
 namespace exact {
 
 __host__ __device__ __forceinline__ int64_t tile_index(int64_t nb, int64_t g, int64_t nbs, int64_t G) {
@@ -78,6 +80,18 @@ __device__ __forceinline__ int64_t floordiv_rcp(int64_t a, int64_t b, double rb)
   while (r < 0) { --q; r += b; }
   while (r >= b) { ++q; r -= b; }
   return q;
+}
+
+// int16 -> (hi, lo - 128) int8 digits of 16 values held in two 16-byte chunks
+__device__ __forceinline__ void split_digits(v4i p0, v4i p1, v4i& hi, v4i& lo) {
+  hi[0] = __builtin_amdgcn_perm(p0[1], p0[0], 0x07050301u);
+  hi[1] = __builtin_amdgcn_perm(p0[3], p0[2], 0x07050301u);
+  hi[2] = __builtin_amdgcn_perm(p1[1], p1[0], 0x07050301u);
+  hi[3] = __builtin_amdgcn_perm(p1[3], p1[2], 0x07050301u);
+  lo[0] = __builtin_amdgcn_perm(p0[1], p0[0], 0x06040200u) ^ 0x80808080;
+  lo[1] = __builtin_amdgcn_perm(p0[3], p0[2], 0x06040200u) ^ 0x80808080;
+  lo[2] = __builtin_amdgcn_perm(p1[1], p1[0], 0x06040200u) ^ 0x80808080;
+  lo[3] = __builtin_amdgcn_perm(p1[3], p1[2], 0x06040200u) ^ 0x80808080;
 }
 
 // SplitMix64 output for counter idx + 1 (Steele, Lea and Flood 2014; exact_llm.py:243-247)

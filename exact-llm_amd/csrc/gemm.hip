@@ -23,7 +23,6 @@
 #include "exact_common.h"
 #include "abi_util.h"
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 #ifndef GEMM_VALU_PER_MFMA

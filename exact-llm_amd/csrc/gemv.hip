@@ -17,8 +17,6 @@
 #include "abi_util.h"
 #include "row_ops.h"
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-
 namespace exact {
 
 __device__ __forceinline__ int sel4(v4i v, int i) {

@@ -10,8 +10,6 @@
 #include "exact_common.h"
 #include "abi_util.h"
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-
 namespace exact {
 
 // one thread per 16-byte (row, 16-k) chunk of the packed tile array

@@ -337,7 +337,7 @@ class TModel:
     def _adds(self, R):
         """{linear of a layer: whether its call on R rows may add into its totals} (ops.linear_adds)"""
         if R not in self._adds_R:
-            L = self.w.layers[0]
+            L = self.w.layers[0] if self.nl else {}
             self._adds_R[R] = {n: ops.linear_adds(R, self.abits, L[n]) for n in ("qkv", "o", "gateup", "down", "router",
                                                                                "sgu", "sd") if n in L}
         return self._adds_R[R]
@@ -524,7 +524,7 @@ class TModel:
                 ops.quant_rows(ws.h, ws.part_sw, c.I // ops.SWIGLU_PART_COLS, self.abits, ws.hq, ws.sh, x8=dh)
                 self._lin(ws.hq, L["down"], t_d, x8=dh)
                 res_t, res_s = t_d, ws.sh
-            elif gsfuse and ops.gemm_swiglu_supported(R, L["gateup"]):   # h takes the place of the totals, which this workspace then never holds
+            elif gsfuse and ops.gemm_swiglu_supported(R, L["gateup"]):   # h takes the place of the totals
                 ops.gemm_swiglu_qrow(dx, L["gateup"], ws.s, tab.silu, t_gu, ws.part_sw, ws.hq, ws.sh, dh)
                 self._lin(ws.hq, L["down"], t_d, x8=dh)
                 res_t, res_s = t_d, ws.sh

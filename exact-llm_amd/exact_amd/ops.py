@@ -408,10 +408,14 @@ def swiglu_qrow(t, s, silu, bits=15, xq=None, sq=None, clear=False, part=None, h
     return xq, sq
 
 
+@functools.lru_cache(maxsize=256)
+def _gemm_swiglu_sizes(R, I, K):
+    return _lib.load().exact_gemm_swiglu_supported(R, I, K) == 1
+
+
 def gemm_swiglu_supported(R, lin):
     """Whether gemm_swiglu_qrow takes R int16 rows of this gate|up linear."""
-    return (lin.mh is None and lin.bias is None and lin.N % 2 == 0
-            and _lib.load().exact_gemm_swiglu_supported(R, lin.N // 2, lin.K) == 1)
+    return lin.mh is None and lin.bias is None and lin.N % 2 == 0 and _gemm_swiglu_sizes(R, lin.N // 2, lin.K)
 
 
 def gemm_swiglu_qrow(x8, lin, s, silu, h, part, xq, sq, xq8=None):
@@ -484,8 +488,8 @@ def attention(qq, sq, cache, slot, pos, expt, out, H, KV, hd, inv, obits=None, n
     Smax = kq.shape[2]
     if obits is not None:
         _need(obits, I32, "obits", R * H)
-    if nkeys is not None and 0 < nkeys <= attention_rows_keys(R, H) and hd in (64, 128) and not any(
-            a.data_ptr() % 16 for a in (qq, kq, v, out)):
+    if nkeys is not None and 0 < nkeys <= attention_rows_keys(R, H) and hd in (64, 128) and not (
+            qq.data_ptr() | kq.data_ptr() | v.data_ptr() | out.data_ptr()) % 16:
         _lib.call("exact_attention_rows", _ptr(qq), _ptr(sq), _ptr(kq), _ptr(sk), _ptr(v), _ptr(slot), _ptr(pos), _ptr(expt),
                   _ptr(out), _ptr(obits), R, H, KV, hd, Smax, nkeys, inv, _stream())
         return out
