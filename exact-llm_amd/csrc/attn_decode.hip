@@ -13,6 +13,8 @@
 //   k_dec_out     the outputs and their bit lengths
 // Together, in a graph: one row of 6002 positions, 28 heads over 4 KV heads, 182 -> 21.4 us (31 MB of keys and values: 6.2 us
 // at the card's copy rate of 4.96 TB/s); 8 rows of 1240 to 1793 positions 112 us in two launches -> 31.8.
+// The grids cover the cache, as a captured launch serves every position: blocks past a row's position leave at once, which at 8 rows
+// of 8 KV heads costs 36 us in a cache of 8192 positions (4096 blocks a launch), so the caller's line counts them.
 #include "exact_common.h"
 #include "abi_util.h"
 

@@ -3,10 +3,10 @@
 // exact_attention takes a 512-thread block per (row, head): of 41 rows' keys at most 41 threads have one, five block barriers
 // order its steps, and 41 rows of 28 heads are 1148 such blocks. Here a wave takes a (row, head): 8 lanes a key make the scores
 // (16-byte loads, whole rows of 256 bytes), after which lane l holds key l of each 64; maximum, exponentials and division are
-// wave reductions, and p.V gives each lane two dimensions, so that a value load is whole rows too. No barrier, 4 waves a block. us a layer of 28 heads over 4 of 128, in a graph,
-// this kernel / exact_attention / the matrix-core kernels: 8 rows 6.2 / 10.1 / -, 41 rows 10.1 / 14.7 / 23.7, 64 rows 12.2 / 21.7 /
-// 24.1, 95 rows 20.4 / 32.1 / 23.8. Bound by the chain of a wave's loads and reductions; a wave that walks four chunks (4 rows at
-// 254 positions) takes 34 against 15.5, so it ends at two.
+// wave reductions, and p.V gives each lane two dimensions, so that a value load is whole rows too. No barrier, 4 waves a block.
+// us a layer of 28 heads over 4 of 128, in a graph, this kernel / exact_attention / the matrix-core kernels: 8 rows 6.2 / 10.1 /
+// -, 41 rows 10.1 / 14.7 / 23.7, 64 rows 12.2 / 21.7 / 24.1, 95 rows 20.4 / 32.1 / 23.8. Bound by the chain of a wave's loads and
+// reductions; a wave that walks four chunks (4 rows at 254 positions) takes 34 against 15.5, so it ends at two.
 #include "exact_common.h"
 #include "abi_util.h"
 

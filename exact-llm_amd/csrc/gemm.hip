@@ -35,7 +35,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 #define GEMM_SMALL_M 128       // rows up to which the 128-row tile configuration runs
 #endif
 #ifndef GEMM_SPLIT_TILES
-#define GEMM_SPLIT_TILES 128   // split K while the output tiles number fewer than this
+#define GEMM_SPLIT_TILES 128   // k_gemm_g128 (gemm_launch) splits K while the output tiles number fewer than this
 #endif
 
 namespace exact {
@@ -560,7 +560,7 @@ namespace exact {
 // a wave are one slice: its bit length of max |h| goes to part[row * I / 32 + slice], and its h to 32 int64 slots of h, as int32
 // in the first half of them when they all fit (bit length <= 31), which halves what the launch stores and the quantising one
 // reads. The totals (two int64 an output) stay in registers: a 7B layer at 1537 rows stored and read back 933 MB of them, 504 us
-// of GEMM and 120 of SwiGLU launch, now 538 (the epilogue's 8192 outputs a block run beside no other block of the CU).
+// of GEMM and 120 of SwiGLU launch, now 511 (the epilogue's 8192 outputs a block run beside no other block of the CU).
 struct SwigluOut {
   const int32_t* s;      // (R) shifts of the GEMM's rows
   const int32_t* silu;

@@ -246,7 +246,6 @@ __global__ __launch_bounds__(SAMPLE_NT) void k_sample_pick(int V, int nch, Sampl
 
 using namespace exact;
 
-
 extern "C" int exact_sample(const int64_t* lg, int32_t R, int32_t V, uint64_t seed, const int32_t* step, int64_t tnum,
                             const int32_t* exp_t, int32_t* ids, int64_t* p_out, void* stream) {
   if (!lg || !step || !exp_t || !ids || R <= 0 || V <= 0 || tnum <= 0) return EXACT_E_ARG;
