@@ -659,17 +659,21 @@ def sample(lg, seed, step, tnum, expt, ids, p_out=None):
     """ids[r] = sample_int(lg[r], seed, step[r], tnum) (exact_llm.py:256-259), on the device."""
     R, V = lg.shape
     seed = ctypes.c_uint64(seed)
-    _need(lg, I64, "lg"), _need(step, I32, "step", R), _need(ids, I32, "ids", R)
+    lgp, stp, idp, pp = _ptr(_need(lg, I64, "lg")), _ptr(_need(step, I32, "step", R)), _ptr(_need(ids, I32, "ids", R)), _ptr(p_out)
     if V < SAMPLE_SPLIT_FROM or (R > SAMPLE_SPLIT_MANY and V < SAMPLE_SPLIT_FROM_MANY):
-        _lib.call("exact_sample", _ptr(lg), R, V, seed, _ptr(step), tnum, _ptr(expt), _ptr(ids), _ptr(p_out), _stream())
+        _lib.call("exact_sample", lgp, R, V, seed, stp, tnum, _ptr(expt), idp, pp, _stream())
         return ids
-    row = _lib.load().exact_sample_workspace(1, V)   # the workspace of n rows is n of these
-    n = max(1, min(R, SAMPLE_WORK_BYTES // row))
-    work = torch.empty(n * row, dtype=I8, device=lg.device)
-    for r in range(0, max(R, 1), n):   # no rows: refused by the call
-        at = lambda t, size: None if t is None else ctypes.c_void_p(t.data_ptr() + r * size)
-        _lib.call("exact_sample_split", at(lg, 8 * V), min(n, R - r), V, seed, at(step, 4), tnum, _ptr(expt), at(ids, 4),
-                  at(p_out, 8 * V), _ptr(work), work.numel(), _stream())
+    need = _lib.load().exact_sample_workspace(R, V)
+    if need <= SAMPLE_WORK_BYTES:
+        work = torch.empty(need, dtype=I8, device=lg.device)
+        _lib.call("exact_sample_split", lgp, R, V, seed, stp, tnum, _ptr(expt), idp, pp, _ptr(work), need, _stream())
+        return ids
+    n = max(1, SAMPLE_WORK_BYTES // (need // R))   # the workspace of n rows is n times one row's
+    work = torch.empty(need // R * n, dtype=I8, device=lg.device)
+    at = lambda p, off: p and ctypes.c_void_p(p.value + off)
+    for r in range(0, R, n):
+        _lib.call("exact_sample_split", at(lgp, 8 * r * V), min(n, R - r), V, seed, at(stp, 4 * r), tnum, _ptr(expt),
+                  at(idp, 4 * r), at(pp, 8 * r * V), _ptr(work), work.numel(), _stream())
     return ids
 
 
