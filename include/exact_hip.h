@@ -326,8 +326,8 @@ int exact_attention_qkv_split(const int64_t* t, const int32_t* s, const int64_t*
 
 /* exact_attention_qkv_split for long caches, as four launches split over the keys (scores, exponentials, p.V, output), so
  * that one row's attention takes more CUs than it has heads and each group of H / KV query heads reads its keys and values
- * once. Same results, cache contents and obits contract. hd 64 or 128,
- * H / KV one of 1, 2, 4, 5, 7, 8, Smax <= 8192 (otherwise EXACT_E_UNSUPPORTED). work: device memory of at least
+ * once. Same results, cache contents and obits contract. hd 64 or 128, H / KV one of 1, 2, 4, 5, 7, 8, Smax <= 8192, kq and v
+ * 16-byte aligned (otherwise EXACT_E_UNSUPPORTED). The grids cover Smax, so few positions in a long cache are faster in one launch. work: device memory of at least
  * exact_attention_decode_workspace(R, H, KV, hd, Smax) bytes (0: sizes the entry point refuses), 256-byte aligned,
  * of this call alone while it runs. Replaces the same steps as exact_attention_qkv (exact_llm.py:170-176). */
 int64_t exact_attention_decode_workspace(int32_t R, int32_t H, int32_t KV, int32_t hd, int32_t Smax);
